@@ -27,8 +27,9 @@
 // added by the norm that follows; gelu is applied as the mlp c_fc product
 // stores its outputs.  The kernels here are the row-wise rest: the
 // embedding, the residual add fused with the next layer norm, and the
-// attention with its cache append (a workgroup of 4 waves per stream and
-// head, 16 when there are few).
+// attention with its cache append (a decode step: a workgroup of 4 waves per
+// stream and head, 16 when there are few; the prompt pass: fp32 matrix-core
+// tiles of 16 rows).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -214,7 +215,6 @@ struct AttnArgs {
     const int32_t* positions;
     const int32_t* act;
     const int32_t* slots;  // prefill: the cache slot of each row (NULL: the row)
-    int32_t appended;      // the rows' k, v already stored (t3_kv_append)
     float* out;            // [n_rows][n_embd]
     uint32_t* parts;       // when set, the rows go there instead, split for the
     float* inv;            //   next product (cbx_split.h), the scales here
@@ -253,13 +253,54 @@ __device__ __forceinline__ void attn_store(const AttnArgs& a, int r, int h, int 
     if (k == 0) a.inv[split_inv_index(T, m, nball, kb)] = sinv;
 }
 
+typedef float mf4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ mf4 mfma_f32(float x, float y, const mf4& acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0);
+}
+
+// Dimensions 4c .. 4c + 3 of head h of row r's attention output from lane c
+// of a 16-lane row (every lane of the wave takes part; nothing stored past
+// n_rows): to out, or split as attn_store does (block 2h + c / 8, its largest
+// magnitude over 8 lanes).
+__device__ __forceinline__ void attn_store4(const AttnArgs& a, int n_rows, int r, int h, int c,
+                                            const mf4& o) {
+    if (!a.parts) {
+        if (r < n_rows)
+            *reinterpret_cast<mf4*>(a.out + (int64_t)r * a.n_head * kHeadDim + h * kHeadDim + 4 * c) = o;
+        return;
+    }
+    float mx = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3])));
+#pragma unroll
+    for (int x = 1; x < 8; x <<= 1) mx = fmaxf(mx, __shfl_xor(mx, x));
+    if (r >= n_rows) return;
+    float sc, sinv;
+    split_scale(mx, sc, sinv);
+    uint32_t hi[2], lo[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float y0 = __fmul_rn(o[2 * i], sc), y1 = __fmul_rn(o[2 * i + 1], sc);
+        const _Float16 h0 = (_Float16)y0, h1 = (_Float16)y1;
+        hi[i] = __builtin_bit_cast(uint32_t, split_h2{h0, h1});
+        lo[i] = __builtin_bit_cast(uint32_t, split_h2{(_Float16)__fsub_rn(y0, (float)h0),
+                                                      (_Float16)__fsub_rn(y1, (float)h1)});
+    }
+    const int nball = a.n_head * kHeadDim / 32, kb = 2 * h + (c >> 3), T = r >> 4, m = r & 15;
+    // values 4 (c % 8) .. of the block: half (c & 1) of group (c % 8) / 2
+    uint32_t* const d =
+        a.parts + ((int64_t)T * nball + kb) * 512 + 4 * (16 * ((c & 7) >> 1) + m) + 2 * (c & 1);
+    *reinterpret_cast<uint2*>(d) = make_uint2(hi[0], hi[1]);
+    *reinterpret_cast<uint2*>(d + 256) = make_uint2(lo[0], lo[1]);
+    if ((c & 7) == 0) a.inv[split_inv_index(T, m, nball, kb)] = sinv;
+}
+
 // Prefill: every row's k and v stored at its slot and position before any
 // row attends, so rows of one stream in one call see each other causally.
 __global__ __launch_bounds__(kHeadDim) void t3_kv_append(AttnArgs a) {
     const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
     if (!a.act[r]) return;
     const int n = a.n_head * kHeadDim;
-    const int slot = a.slots ? a.slots[r] : r, pos = a.positions[r];
+    const int slot = a.slots[r], pos = a.positions[r];
     const float* qr = a.qkv + (int64_t)r * 3 * n + h * kHeadDim;
     const int64_t base =
         (((int64_t)slot * a.n_layer + a.layer) * a.n_head + h) * a.n_ctx * kHeadDim + (int64_t)pos * kHeadDim;
@@ -274,12 +315,9 @@ __global__ __launch_bounds__(kHeadDim) void t3_kv_append(AttnArgs a) {
 // per load instruction, kAttnBatch rows per lane in flight, and go over the
 // run once with a running softmax (max, sum, weighted v sums, rescaled as the
 // max grows); the runs of the 4 row groups of a wave and of the waves are
-// merged by the same rescaling in a fixed order.  Decode steps run 4 waves x
-// 6 rows (every workgroup resident at once; 16 waves when rows x heads are
-// under 256, see t3_attn_wide), the prompt pass 2 waves x 8 rows
-// (many more workgroups: smaller ones keep more of them resident); measured
-// at 64 streams 1.89 -> 1.85 ms per step against 4 x 8, and the prompt of
-// 64 x 256 positions 93.8 -> 82.2 ms.
+// merged by the same rescaling in a fixed order.  4 waves x 6 rows (every
+// workgroup resident at once; 16 waves when rows x heads are under 256, see
+// t3_attn_wide); measured at 64 streams 1.89 -> 1.85 ms per step against 4 x 8.
 template <int kAttnBatch, int kAttnWaves>
 __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
     __shared__ __align__(16) float kn_s[kHeadDim];
@@ -294,17 +332,14 @@ __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
         return;
     }
     const int pos = a.positions[r];
-    const int slot = a.slots ? a.slots[r] : r;
     const float* qr = a.qkv + (int64_t)r * 3 * n + h * kHeadDim;
-    const int64_t base = (((int64_t)slot * a.n_layer + a.layer) * a.n_head + h) * a.n_ctx * kHeadDim;
+    const int64_t base = (((int64_t)r * a.n_layer + a.layer) * a.n_head + h) * a.n_ctx * kHeadDim;
     float* kc = a.kc + base;
     float* vc = a.vc + base;
     if (w == 0) {
         const float kn = qr[n + lane], vn = qr[2 * n + lane];
-        if (!a.appended) {
-            kc[(int64_t)pos * kHeadDim + lane] = kn;
-            vc[(int64_t)pos * kHeadDim + lane] = vn;
-        }
+        kc[(int64_t)pos * kHeadDim + lane] = kn;
+        vc[(int64_t)pos * kHeadDim + lane] = vn;
         kn_s[lane] = kn;
         vn_s[lane] = vn;
     }
@@ -410,9 +445,240 @@ __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
     }
 }
 
+// The prompt pass's attention on the fp32 matrix cores: a wave takes 16
+// consecutive rows of one head and walks their stream's positions in tiles
+// of 16, so a tile of K and V is read once for all its rows (a workgroup per
+// row read both again for every row, which bound it).
+// v_mfma_f32_16x16x4_f32 throughout: products and sums in binary32.
+//  * Scores transposed, S^T = K Q^T: lane (g = l/16, c = l%16) feeds K row c
+//    and Q row c at dimensions 16 cc + 4 g + e (step (cc, e); the four lane
+//    groups of a step supply its four dimensions, any order), and holds the
+//    scores of row c at keys 4 g + v: its own row's mask, maximum and sum,
+//    joined over g by two exchanges.
+//  * P V: those scores' exponentials are the A operand as they stand (row c,
+//    step v: key 4 g + v), V[4 g + v][4 c ..] the B operand, one 16-byte load
+//    for four output tiles (tile dt, column c: dimension 4 c + dt), so lane
+//    (g, c) ends with rows 4 g + v at dimensions 4 c .. 4 c + 3.
+// Each row has its running max, sum and outputs (rescaled as its max grows;
+// a tile in which a row sees no key leaves that row's as they are), so a
+// row's result does not depend on the rows beside it.  The 16 rows may belong
+// to any slots: one pass per distinct slot, the other rows' keys masked.
+// A masked key's weight is 0, and 0 times a V that is not finite would reach
+// rows that do not see that key: tiles that some row does not see whole look
+// for such values and, where one is found, add row by row with the unseen
+// keys' V at 0.
+// KS = 4: the workgroup's four waves take the same rows and every fourth
+// pair of tiles, merged through LDS by the same rescaling in wave order
+// (small calls); KS = 1: each wave its own rows.
+// Measured per layer at 64 prompts of 129 to 383 rows (14975 in all), 16
+// heads: 1051 -> 200 us (matrix cores busy 42% of it; they alone would take
+// about 80); one prompt of 251 rows 24.5 -> 11 us.  32 rows per wave (half the
+// loads of K and V) measured 235: registers for two waves per SIMD, not three.
+template <int KS>
+__global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_rows) {
+    constexpr int kWaves = 4, KT = 2;  // KT tiles of 16 keys per iteration
+    static_assert(KS == 1 || KS == kWaves, "every wave its own rows, or all the same");
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int g = lane >> 4, c = lane & 15, h = blockIdx.y;
+    const int n = a.n_head * kHeadDim;
+    const int r0 = (KS == 1 ? (int)blockIdx.x * kWaves + w : (int)blockIdx.x) * 16;
+    if (r0 >= n_rows) return;  // whole waves, and only where no barrier follows (KS = 1)
+    const int rc = min(r0 + c, n_rows - 1);
+    const bool real = r0 + c < n_rows && a.act[rc] != 0;
+    const int pos = a.positions[rc], slot = a.slots[rc];
+    mf4 q[4], o[4];
+    {
+        const float* const qr = a.qkv + (int64_t)rc * 3 * n + h * kHeadDim + 4 * g;
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+            q[cc] = *reinterpret_cast<const mf4*>(qr + 16 * cc);
+            o[cc] = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    float m = -INFINITY, s = 0.0f;
+    bool todo = real;
+    for (;;) {
+        // the first row still to do names the pass's slot
+        const uint64_t left = __ballot(todo);
+        if (!left) break;
+        const int cur = __builtin_amdgcn_readlane(slot, (int)__builtin_ctzll(left));
+        // lim: the last position the row sees in this pass (-1: none); last
+        // over the rows, least over the group's active rows
+        const bool now = todo && slot == cur;
+        todo = todo && !now;
+        const int lim = now ? pos : -1;
+        int last = lim, least = real ? lim : INT32_MAX;
+#pragma unroll
+        for (int x = 1; x < 16; x <<= 1) {
+            last = max(last, __shfl_xor(last, x));
+            least = min(least, __shfl_xor(least, x));
+        }
+        last = __builtin_amdgcn_readfirstlane(last);
+        least = __builtin_amdgcn_readfirstlane(least);
+        const int64_t base =
+            (((int64_t)cur * a.n_layer + a.layer) * a.n_head + h) * a.n_ctx * kHeadDim;
+        const float* const kc = a.kc + base;
+        const float* const vc = a.vc + base;
+        for (int j0 = KS == 1 ? 0 : 16 * KT * w; j0 <= last; j0 += 16 * KT * KS) {
+            // keys past the last read the last one's row, at weight 0
+            mf4 kk[KT][4], vv[KT][4], p[KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                const float* const kr =
+                    kc + (int64_t)min(j0 + 16 * kt + c, last) * kHeadDim + 4 * g;
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc)
+                    kk[kt][cc] = *reinterpret_cast<const mf4*>(kr + 16 * cc);
+            }
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    vv[kt][v] = *reinterpret_cast<const mf4*>(
+                        vc + (int64_t)min(j0 + 16 * kt + 4 * g + v, last) * kHeadDim + 4 * c);
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) p[kt] = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int kt = 0; kt < KT; ++kt)
+                        p[kt] = mfma_f32(kk[kt][cc][e], q[cc][e], p[kt]);
+            float bm = -INFINITY;
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    p[kt][v] = __fmul_rn(p[kt][v], a.scale);
+                    if (j0 + 16 * kt + 4 * g + v <= lim) bm = fmaxf(bm, p[kt][v]);
+                }
+            bm = fmaxf(bm, __shfl_xor(bm, 16));
+            bm = fmaxf(bm, __shfl_xor(bm, 32));
+            if (__ballot(bm > m)) {
+                const float nm = fmaxf(m, bm);
+                const float f = m == -INFINITY ? 0.0f : expf(__fsub_rn(m, nm));
+                s = __fmul_rn(s, f);
+                m = nm;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float fv = __shfl(f, 4 * g + v);  // row 4 g + v's
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) o[dt][v] = __fmul_rn(o[dt][v], fv);
+                }
+            }
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const bool seen = j0 + 16 * kt + 4 * g + v <= lim;
+                    p[kt][v] = seen ? expf(__fsub_rn(p[kt][v], m)) : 0.0f;
+                    s = __fadd_rn(s, p[kt][v]);
+                }
+            bool plain = true;
+            if (j0 + 16 * KT - 1 > least) {
+                float z = 0.0f;  // NaN once a value is not finite
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+#pragma unroll
+                        for (int dt = 0; dt < 4; ++dt) z = __fmaf_rn(vv[kt][v][dt], 0.0f, z);
+                plain = __ballot(z != z) == 0;
+            }
+            if (plain) {
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+#pragma unroll
+                        for (int dt = 0; dt < 4; ++dt)
+                            o[dt] = mfma_f32(p[kt][v], vv[kt][v][dt], o[dt]);
+            } else {
+#pragma unroll 1
+                for (int i = 0; i < 16; ++i) {
+                    const int li = __builtin_amdgcn_readlane(lim, i);
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) {
+                        mf4 add = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) {
+                                const bool seen = j0 + 16 * kt + 4 * g + v <= li;
+                                add = mfma_f32(p[kt][v], seen ? vv[kt][v][dt] : 0.0f, add);
+                            }
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (4 * g + v == i) o[dt][v] = __fadd_rn(o[dt][v], add[v]);
+                    }
+                }
+            }
+        }
+    }
+    s = __fadd_rn(s, __shfl_xor(s, 16));  // the row's sum over its four lanes
+    s = __fadd_rn(s, __shfl_xor(s, 32));
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float sv = __shfl(s, 4 * g + v);
+            const bool on = __shfl((int)real, 4 * g + v) != 0;
+            mf4 x;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) x[dt] = on ? __fdiv_rn(o[dt][v], sv) : 0.0f;
+            attn_store4(a, n_rows, r0 + 4 * g + v, h, c, x);
+        }
+    } else {
+        // wave w joins the four waves' rows 4 g + w
+        __shared__ mf4 os[KS][4][64];
+        __shared__ float ms[KS][16], ss[KS][16];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) os[w][v][lane] = mf4{o[0][v], o[1][v], o[2][v], o[3][v]};
+        if (g == 0) {
+            ms[w][c] = m;
+            ss[w][c] = s;
+        }
+        __syncthreads();
+        const int i = 4 * g + w;
+        float M = ms[0][i];
+#pragma unroll
+        for (int x = 1; x < KS; ++x) M = fmaxf(M, ms[x][i]);
+        float st = 0.0f;
+        mf4 at = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int x = 0; x < KS; ++x) {
+            const float f = ms[x][i] == -INFINITY ? 0.0f : expf(__fsub_rn(ms[x][i], M));
+            st = __fadd_rn(st, __fmul_rn(ss[x][i], f));
+            const mf4 ov = os[x][w][lane];
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) at[dt] = __fadd_rn(at[dt], __fmul_rn(ov[dt], f));
+        }
+        const bool on = __shfl((int)real, i) != 0;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) at[dt] = on ? __fdiv_rn(at[dt], st) : 0.0f;
+        attn_store4(a, n_rows, r0 + i, h, c, at);
+    }
+}
+
 template <int EPT>
 hipError_t launch_norm_ept(const NormArgs& a, int n_rows, hipStream_t st) {
     hipLaunchKernelGGL(t3_norm<EPT>, dim3((unsigned)n_rows), dim3(kNormThreads), 0, st, a);
+    return hipGetLastError();
+}
+
+// One 16-row group per wave, or four waves per group (KS = 4) while the
+// groups would not give every SIMD (1024) a wave.  ms per prompt pass, KS = 4 /
+// KS = 1: 1 x 251 rows 1.91 / 2.23, 1 x 700 3.77 / 4.29, 4 x 251 (1008 groups)
+// 4.49 / 4.53, 64 x 24 (1536) 6.10 / 5.90, 16 x 251 14.48 / 14.43, 48 x 290
+// 50.6 / 50.0.
+hipError_t launch_attn_tile(const AttnArgs& a, int n_rows, hipStream_t st) {
+    const int groups = (n_rows + 15) / 16;
+    if ((int64_t)groups * a.n_head < 1024)
+        hipLaunchKernelGGL(t3_attn_tile<4>, dim3((unsigned)groups, (unsigned)a.n_head),
+                           dim3(4 * kHeadDim), 0, st, a, n_rows);
+    else
+        hipLaunchKernelGGL(t3_attn_tile<1>, dim3((unsigned)((groups + 3) / 4), (unsigned)a.n_head),
+                           dim3(4 * kHeadDim), 0, st, a, n_rows);
     return hipGetLastError();
 }
 
@@ -523,7 +789,6 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     aa.positions = positions;
     aa.act = act;
     aa.slots = slots;
-    aa.appended = prefill ? 1 : 0;
     aa.out = att;
     aa.parts = mc ? sparts : nullptr;  // c_attn has read them by then
     aa.inv = sinv;
@@ -565,16 +830,14 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
             hipLaunchKernelGGL(t3_kv_append, dim3((unsigned)n_rows, (unsigned)m.n_head),
                                dim3(kHeadDim), 0, st, aa);
             if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        if (prefill)
-            hipLaunchKernelGGL((t3_attn<8, 2>), dim3((unsigned)n_rows, (unsigned)m.n_head),
-                               dim3(2 * kHeadDim), lds, st, aa);
-        else if (wide)
+            if ((e = launch_attn_tile(aa, n_rows, st)) != hipSuccess) return e;
+        } else if (wide) {
             hipLaunchKernelGGL((t3_attn<6, 16>), dim3((unsigned)n_rows, (unsigned)m.n_head),
                                dim3(16 * kHeadDim), lds, st, aa);
-        else
+        } else {
             hipLaunchKernelGGL((t3_attn<6, 4>), dim3((unsigned)n_rows, (unsigned)m.n_head),
                                dim3(4 * kHeadDim), lds, st, aa);
+        }
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // the two products the residual adds take a K split when their grid
         // is narrow (the norm adds the slabs)

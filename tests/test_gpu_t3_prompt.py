@@ -1,0 +1,158 @@
+"""GPU parity of the prompt pass's attention tiles (t3_attn_tile,
+chatterbox.cpp_amd/csrc/cbx_t3.hip) against the binary64 oracle's prompt
+graph, on a small model (2 layers, n_embd 256, 4 heads of 64) so that the row
+counts can take every edge: 16-row groups with one row, whole and one over,
+several streams in one group, keys ending inside and at the edge of a pair of
+16-key tiles, and both forms (a group per wave, or its keys split over four
+waves).
+
+Tolerance on ln_f's rows: |gpu - ref| <= 5e-5 + 5e-5 |ref|, the step tests'
+(tests/test_gpu_t3.py): binary32 throughout against binary64, values O(1),
+fewer layers here.
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import pkg
+from oracle import cbx_t3_oracle as T3
+
+pytestmark = pytest.mark.gpu
+
+L_, N, H, N_POS, V = 2, 256, 4, 512, 64
+TOL_ABS, TOL_REL = 5e-5, 5e-5
+
+
+@pytest.fixture(scope="module")
+def small():
+    import torch
+    assert torch.cuda.is_available(), "GPU tests need a visible MI355X"
+    mod = pkg.load()
+    s = mod.Sampler(device=0, max_vocab=1024, max_history=64)
+    rng = np.random.default_rng(0x9A11)
+    t = lambda a: torch.from_numpy(a).cuda()
+    vec = lambda k, base=0.0, sd=0.1: (base + rng.standard_normal(k) * sd).astype(np.float32)
+    dev, ref = [], []
+    for _ in range(L_):
+        d, r = {}, {}
+        for key, o, i in (("attn_w", 3, 1), ("attn_proj_w", 1, 1), ("fc_w", 4, 1),
+                          ("fc_proj_w", 1, 4)):
+            # large enough that some scores stand out: the running max grows
+            w = (rng.standard_normal((o * N, i * N)) * 0.08).astype(np.float32)
+            blocks = O.quantize(w, O.WTYPE_Q8_0)
+            d[key], r[key] = t(blocks.reshape(-1)), O.dequantize(blocks, O.WTYPE_Q8_0, i * N)
+        for key, k, base in (("ln_1_g", N, 1.0), ("ln_1_b", N, 0.0), ("attn_b", 3 * N, 0.0),
+                             ("attn_proj_b", N, 0.0), ("ln_2_g", N, 1.0), ("ln_2_b", N, 0.0),
+                             ("fc_b", 4 * N, 0.0), ("fc_proj_b", N, 0.0)):
+            r[key] = vec(k, base)
+            d[key] = t(r[key])
+        dev.append(d)
+        ref.append(r)
+    wpe, emb, gf, bf = vec((N_POS, N)), vec((V, N), 0.0, 0.5), vec(N, 1.0), vec(N)
+    dm = mod.Sampler.t3_model(dev, t(wpe), t(emb), t(gf), t(bf), wtype=O.WTYPE_Q8_0, n_head=H)
+    yield torch, s, dm, T3.Model(ref, wpe, emb, gf, bf, 1e-5, H)
+    s.close()
+
+
+def run(torch, s, dm, rows, inputs, n_slots, n_ctx, caches=None):
+    """rows: (slot, position) of each input row.  Caches start as NaN (what
+    was never stored must never be used) unless given."""
+    if caches is None:
+        k = torch.full((n_slots, L_, H, n_ctx, 64), float("nan"), device="cuda")
+        caches = (k, k.clone())
+    k, v = caches
+    hid = torch.full((len(rows), N), 7.0, device="cuda")
+    at = np.array(rows, np.int32)
+    s.t3_prefill(dm, torch.from_numpy(at[:, 0].copy()).cuda(),
+                 torch.from_numpy(at[:, 1].copy()).cuda(), k, v, hid,
+                 inputs=torch.from_numpy(inputs).cuda())
+    torch.cuda.synchronize()
+    return hid.cpu().numpy(), k, v
+
+
+def arranged(lens, order, rng):
+    rows = [(b, p) for b, n in enumerate(lens) for p in range(n)]
+    if order == "positions":   # every stream's first row, then every second ...
+        rows.sort(key=lambda x: (x[1], x[0]))
+    elif order == "shuffled":
+        rows = [rows[i] for i in rng.permutation(len(rows))]
+    return rows
+
+
+CASES = [
+    ((1,), "streams"), ((16,), "streams"), ((17,), "streams"), ((31,), "streams"),
+    ((32,), "streams"), ((33, 1, 64, 127), "streams"), ((5, 40, 18), "positions"),
+    ((70, 9, 33), "shuffled"), ((251,), "streams"),
+    ((250, 129, 383) + (61,) * 60, "streams"),   # 4422 rows: a group per wave
+    ((65,) * 64, "positions"),                   # 4160 rows, 16 streams in a group
+]
+
+
+@pytest.mark.parametrize("lens,order", CASES, ids=[f"{sum(c[0])}-{c[1]}" for c in CASES])
+def test_prompt_rows_match_oracle(small, lens, order):
+    """Every row and every stored key and value, some rows of each call being
+    skipped ones (slot or position out of range), which give zero rows."""
+    torch, s, dm, rm = small
+    rng = np.random.default_rng(sum(lens) + len(order))
+    rows = arranged(lens, order, rng)
+    skip = set(rng.integers(0, len(rows) + 1, 3).tolist()) if len(rows) > 16 else set()
+    for at in sorted(skip, reverse=True):
+        rows.insert(at, [(-1, 0), (len(lens), 1), (0, 400)][at % 3])
+    x = (rng.standard_normal((len(rows), N)) * 0.7).astype(np.float32)
+    print(f"[gpu-case] prompt lens={lens[:4]} order={order} rows={len(rows)}", flush=True)
+    got, k, v = run(torch, s, dm, rows, x, len(lens), 400)
+    kr, vr = T3.new_cache(len(lens), L_, H, 400)
+    where = {key: i for i, key in enumerate(rows)}
+    for b, n in enumerate(lens):
+        at = [where[(b, p)] for p in range(n)]
+        want = T3.prefill(rm, x[at], kr, vr, b, 0)
+        err = np.abs(got[at] - want)
+        assert np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), f"stream {b}: {err.max():.3g}"
+        for c, r in ((k, kr), (v, vr)):
+            c = c[b, :, :, :n].cpu().numpy()
+            assert np.allclose(c, r[b, :, :, :n], rtol=TOL_REL, atol=TOL_ABS)
+    good = {(b, p) for b, n in enumerate(lens) for p in range(n)}
+    for i, key in enumerate(rows):
+        if key not in good:
+            assert np.all(got[i] == 0.0)
+
+
+def test_rows_independent_of_the_rows_beside_them(small):
+    """A stream's rows are bit for bit the same alone, beside others and in
+    another order (both with four waves per group)."""
+    torch, s, dm, _ = small
+    rng = np.random.default_rng(7)
+    x = {(b, p): (rng.standard_normal(N) * 0.7).astype(np.float32)
+         for b in range(3) for p in range(60)}
+    out = {}
+    for name, rows in (("alone", [(0, p) for p in range(60)]),
+                       ("beside", arranged((60, 60, 60), "streams", rng)),
+                       ("shuffled", arranged((60, 60, 60), "shuffled", rng))):
+        print(f"[gpu-case] independence {name}", flush=True)
+        got, _, _ = run(torch, s, dm, rows, np.stack([x[r] for r in rows]), 3, 64)
+        out[name] = np.stack([got[rows.index((0, p))] for p in range(60)])
+    assert np.array_equal(out["alone"], out["beside"])
+    assert np.array_equal(out["alone"], out["shuffled"])
+
+
+@pytest.mark.parametrize("lens", [(40, 21), (70,) * 60], ids=["split-keys", "group-per-wave"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_nonfinite_row_stays_in_its_stream(small, lens, bad):
+    """One prompt row that is not finite: the rows before it and the other
+    streams' (in the same group) are what they are without it, bit for bit;
+    the row itself and those after it are not finite."""
+    torch, s, dm, _ = small
+    rng = np.random.default_rng(11)
+    rows = arranged(lens, "positions", rng)
+    x = (rng.standard_normal((len(rows), N)) * 0.7).astype(np.float32)
+    print(f"[gpu-case] nonfinite {bad} rows={len(rows)}", flush=True)
+    clean, _, _ = run(torch, s, dm, rows, x, len(lens), 80)
+    hit = (1, 18)
+    y = x.copy()
+    y[rows.index(hit), 3] = bad
+    got, _, _ = run(torch, s, dm, rows, y, len(lens), 80)
+    for i, (b, p) in enumerate(rows):
+        if b == hit[0] and p >= hit[1]:
+            assert np.isnan(got[i]).any()
+        else:
+            assert np.array_equal(got[i], clean[i]), (b, p)
