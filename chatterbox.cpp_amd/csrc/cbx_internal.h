@@ -156,6 +156,16 @@ hipError_t launch_head_presplit(const void* W, int32_t wtype, const float* bias,
                                 const void* scratch, hipStream_t stream, int kz,
                                 bool gelu_out, void* out_split = nullptr);
 
+// The same for many rows (cbx_tile.hip; head_uses_tiles: the rows and widths it
+// takes): the weights unpacked into `scratch` (device memory of
+// tile_scratch_bytes) for the call, then tiles bound by the matrix cores.
+bool head_uses_tiles(int32_t n_rows, int32_t n_embd);
+size_t tile_scratch_bytes(int32_t n_rows, int32_t n_vocab, int32_t n_embd);
+hipError_t launch_head_tiles(const void* W, int32_t wtype, const float* bias, float* out,
+                             int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
+                             const void* split, void* scratch, hipStream_t stream, bool gelu_out,
+                             void* out_split);
+
 // The T3 layer's residual add and layer norm folded into the mat-vec product
 // that consumes them (1 or 2 rows of n_embd, a multiple of 256, at most
 // 4096): per row r, x_out[r] = x_in[r] + y[r], and the product's input row is

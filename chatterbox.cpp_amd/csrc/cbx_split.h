@@ -55,12 +55,23 @@ __device__ __forceinline__ void split_store(uint32_t* parts, int T, int m, int n
 }
 
 // The T3 MLP's gelu, tanh form (Hendrycks and Gimpel; ggml_gelu's):
-// 0.5 x (1 + tanh(sqrt(2/pi) x (1 + 0.044715 x^2))), each operation rounded.
+// 0.5 x (1 + tanh(w)) with w = sqrt(2/pi) x (1 + 0.044715 x^2), taken as
+// x / (1 + exp(-2 w)), which is the same function without the cancellation
+// of 1 + tanh(w) at negative w.  exp through 2^t, t = -2 w log2(e), with the
+// rounding of t carried (an error of t is one of the whole result, |t| times
+// over); t is bounded where 2^t is 0 or infinite anyway, so that the
+// remainder stays finite.  About 20 instructions (tanhf: about 60), the
+// largest part of a c_fc tile's end.
 __device__ __forceinline__ float t3_gelu_f(float x) {
     const float c = 0.7978845608028654f;  // sqrt(2 / pi)
-    const float inner =
+    const float kL = -2.8853900817779268f, kLlo = -2.8853900817779268 - (double)-2.8853900817779268f;
+    const float w =
         __fmul_rn(__fmul_rn(c, x), __fadd_rn(1.0f, __fmul_rn(__fmul_rn(0.044715f, x), x)));
-    return __fmul_rn(__fmul_rn(0.5f, x), __fadd_rn(1.0f, tanhf(inner)));
+    const float wc = fminf(fmaxf(w, -60.0f), 60.0f);  // t within +-174
+    const float t = __fmul_rn(wc, kL);
+    const float r = __fmaf_rn(wc, kLlo, __fmaf_rn(wc, kL, -t));
+    const float e = __fmul_rn(__builtin_amdgcn_exp2f(t), __fmaf_rn(r, 0.6931471805599453f, 1.0f));
+    return __fmul_rn(x, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, e)));
 }
 
 // A DPP lane exchange within each 16-lane row (ctrl a compile-time DPP code).
@@ -82,6 +93,21 @@ __device__ __forceinline__ float sum16_dpp(float v) {
     v = __fadd_rn(v, dpp16<0x4E>(v));   // quad_perm [2, 3, 0, 1]
     v = __fadd_rn(v, dpp16<0x141>(v));  // row_half_mirror
     return __fadd_rn(v, dpp16<0x140>(v));  // row_mirror
+}
+
+// The largest of v (no NaN matters: fmaxf) over each 16-lane row, the same in
+// every lane of it, by the same exchanges.
+__device__ __forceinline__ float max16_dpp(float v) {
+    v = fmaxf(v, dpp16<0xB1>(v));
+    v = fmaxf(v, dpp16<0x4E>(v));
+    v = fmaxf(v, dpp16<0x141>(v));
+    return fmaxf(v, dpp16<0x140>(v));
+}
+
+// A scaled value y's two fp16 parts, hi in the low half.
+__device__ __forceinline__ uint32_t split_pair(float y) {
+    const _Float16 h = (_Float16)y;
+    return __builtin_bit_cast(uint32_t, split_h2{h, (_Float16)__fsub_rn(y, (float)h)});
 }
 
 // Sum of one value per thread over a workgroup of 256 threads, the same

@@ -717,14 +717,16 @@ bool t3_attn_wide(int32_t n_rows, int32_t n_head) { return (int64_t)n_rows * n_h
 // qkv [n_rows][3 n_embd], f [n_rows][4 n_embd], act [n_rows], then two
 // buffers of split activations for the matrix products (each for the widest
 // input, 4 n_embd): the norms and the attention write the first, the mlp's
-// c_fc the second (c_fc reads the first as it writes).
+// c_fc the second (c_fc reads the first as it writes), then, where the rows are
+// many (head_uses_tiles), the largest matrix unpacked for its product.
 
 size_t t3_workspace_bytes(int32_t n_rows, int32_t n_embd) {
     const size_t row = (size_t)n_rows * n_embd * 4;
     const size_t body = (3 + kMaxKSplit) * row + 3 * row + 4 * row +
                         ((size_t)n_rows * 4 + 255) / 256 * 256;
     const size_t sp = (head_scratch_bytes(n_rows, false, 4 * n_embd) + 255) / 256 * 256;
-    return body + 2 * sp;
+    return body + 2 * sp + max(tile_scratch_bytes(n_rows, 4 * n_embd, n_embd),
+                               tile_scratch_bytes(n_rows, n_embd, 4 * n_embd));
 }
 
 hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* tokens,
@@ -747,6 +749,8 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     void* split = reinterpret_cast<char*>(act) + ((size_t)n_rows * 4 + 255) / 256 * 256;
     void* split2 = static_cast<char*>(split) +
                    (head_scratch_bytes(n_rows, false, 4 * n) + 255) / 256 * 256;
+    void* unpacked = static_cast<char*>(split2) +
+                     (head_scratch_bytes(n_rows, false, 4 * n) + 255) / 256 * 256;
 
     NormArgs na{};
     na.n_embd = n;
@@ -808,11 +812,19 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     gn.y = y;
     gn.act = act;
     gn.eps = m.eps;
+    // the products of rows already split, from `in`
+    auto product = [&](const void* w, const float* b, float* out, int n_out, int n_in,
+                       const void* in, int kz, bool gelu, void* out_split) {
+        return head_uses_tiles(n_rows, n_in) && kz == 1
+                   ? launch_head_tiles(w, m.wtype, b, out, n_out, n_rows, n_out, n_in, in, unpacked,
+                                       st, gelu, out_split)
+                   : launch_head_presplit(w, m.wtype, b, out, n_out, n_rows, n_out, n_in, in, st,
+                                          kz, gelu, out_split);
+    };
     for (int l = 0; l < m.n_layer; ++l) {
         const cbx_t3_layer& L = m.layers[l];
         if (mc) {
-            e = launch_head_presplit(L.attn_w, m.wtype, L.attn_b, qkv, 3 * n, n_rows, 3 * n, n,
-                                     split, st, 1, false);
+            e = product(L.attn_w, L.attn_b, qkv, 3 * n, n, split, 1, false, nullptr);
         } else if (fold && l > 0) {  // the previous layer's residual + this ln_1
             gn.x_in = xcur;
             gn.x_out = xcur = xcur == x ? xalt : x;
@@ -841,8 +853,7 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // the two products the residual adds take a K split when their grid
         // is narrow (the norm adds the slabs)
-        e = mc ? launch_head_presplit(L.attn_proj_w, m.wtype, L.attn_proj_b, y, n, n_rows, n, n,
-                                      split, st, kz_a, false)
+        e = mc ? product(L.attn_proj_w, L.attn_proj_b, y, n, n, split, kz_a, false, nullptr)
                : launch_head_k(L.attn_proj_w, m.wtype, L.attn_proj_b, att, nullptr, n, y, nullptr,
                                n, n_rows, n, n, split, st, kz_a, false);
         if (e != hipSuccess) return e;
@@ -869,14 +880,12 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
                                       true);
         } else {
             if ((e = launch_norm(nb, n_rows, st)) != hipSuccess) return e;
-            e = mc ? launch_head_presplit(L.fc_w, m.wtype, L.fc_b, f, 4 * n, n_rows, 4 * n, n,
-                                          split, st, 1, true, split2)
+            e = mc ? product(L.fc_w, L.fc_b, f, 4 * n, n, split, 1, true, split2)
                    : launch_head_k(L.fc_w, m.wtype, L.fc_b, u, nullptr, n, f, nullptr, 4 * n,
                                    n_rows, 4 * n, n, split, st, 1, true);
         }
         if (e != hipSuccess) return e;
-        e = mc ? launch_head_presplit(L.fc_proj_w, m.wtype, L.fc_proj_b, y, n, n_rows, n, 4 * n,
-                                      split2, st, kz_f, false)
+        e = mc ? product(L.fc_proj_w, L.fc_proj_b, y, n, 4 * n, split2, kz_f, false, nullptr)
                : launch_head_k(L.fc_proj_w, m.wtype, L.fc_proj_b, f, nullptr, 4 * n, y, nullptr, n,
                                n_rows, n, 4 * n, split, st, kz_f, false);
         if (e != hipSuccess) return e;

@@ -29,6 +29,11 @@ def small():
     assert torch.cuda.is_available(), "GPU tests need a visible MI355X"
     mod = pkg.load()
     s = mod.Sampler(device=0, max_vocab=1024, max_history=64)
+    yield (torch, s) + model(torch, mod, O.WTYPE_Q8_0)
+    s.close()
+
+
+def model(torch, mod, wtype):
     rng = np.random.default_rng(0x9A11)
     t = lambda a: torch.from_numpy(a).cuda()
     vec = lambda k, base=0.0, sd=0.1: (base + rng.standard_normal(k) * sd).astype(np.float32)
@@ -39,8 +44,8 @@ def small():
                           ("fc_proj_w", 1, 4)):
             # large enough that some scores stand out: the running max grows
             w = (rng.standard_normal((o * N, i * N)) * 0.08).astype(np.float32)
-            blocks = O.quantize(w, O.WTYPE_Q8_0)
-            d[key], r[key] = t(blocks.reshape(-1)), O.dequantize(blocks, O.WTYPE_Q8_0, i * N)
+            blocks = O.quantize(w, wtype)
+            d[key], r[key] = t(blocks.reshape(-1)), O.dequantize(blocks, wtype, i * N)
         for key, k, base in (("ln_1_g", N, 1.0), ("ln_1_b", N, 0.0), ("attn_b", 3 * N, 0.0),
                              ("attn_proj_b", N, 0.0), ("ln_2_g", N, 1.0), ("ln_2_b", N, 0.0),
                              ("fc_b", 4 * N, 0.0), ("fc_proj_b", N, 0.0)):
@@ -49,9 +54,8 @@ def small():
         dev.append(d)
         ref.append(r)
     wpe, emb, gf, bf = vec((N_POS, N)), vec((V, N), 0.0, 0.5), vec(N, 1.0), vec(N)
-    dm = mod.Sampler.t3_model(dev, t(wpe), t(emb), t(gf), t(bf), wtype=O.WTYPE_Q8_0, n_head=H)
-    yield torch, s, dm, T3.Model(ref, wpe, emb, gf, bf, 1e-5, H)
-    s.close()
+    dm = mod.Sampler.t3_model(dev, t(wpe), t(emb), t(gf), t(bf), wtype=wtype, n_head=H)
+    return dm, T3.Model(ref, wpe, emb, gf, bf, 1e-5, H)
 
 
 def run(torch, s, dm, rows, inputs, n_slots, n_ctx, caches=None):
@@ -156,3 +160,30 @@ def test_nonfinite_row_stays_in_its_stream(small, lens, bad):
             assert np.isnan(got[i]).any()
         else:
             assert np.array_equal(got[i], clean[i]), (b, p)
+
+
+# 1024 rows is where the products take large tiles; 8 x 1025 rows give c_attn
+# and c_fc (768 and 1024 outputs) enough workgroups of 128 x 128, attn c_proj not
+@pytest.mark.parametrize("wtype,lens", [
+    (O.WTYPE_Q4_0, (64,) * 16), (O.WTYPE_F16, (37,) * 30), (O.WTYPE_Q5_0, (1,) * 1023 + (18,)),
+    (O.WTYPE_Q8_0, (100,) * 82), (O.WTYPE_F16, (410,) * 20), (O.WTYPE_Q4_0, (391,) * 21)])
+def test_many_rows_products(small, wtype, lens):
+    """The tiled products, every format, whole and partial row tiles."""
+    torch, s = small[:2]
+    dm, rm = model(torch, pkg.load(), wtype)
+    rng = np.random.default_rng(len(lens))
+    rows = arranged(lens, "streams", rng)
+    x = (rng.standard_normal((len(rows), N)) * 0.7).astype(np.float32)
+    print(f"[gpu-case] many rows wtype={wtype} rows={len(rows)}", flush=True)
+    got, k, v = run(torch, s, dm, rows, x, len(lens), max(lens) + 1)
+    at = 0
+    for b, n in enumerate(lens):
+        if b % 5 == 0 or b + 1 == len(lens):
+            kr, vr = T3.new_cache(1, L_, H, n)
+            want = T3.prefill(rm, x[at:at + n], kr, vr, 0, 0)
+            err = np.abs(got[at:at + n] - want)
+            assert np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), f"stream {b}: {err.max():.3g}"
+            for c, r in ((k, kr), (v, vr)):
+                assert np.allclose(c[b, :, :, :n].cpu().numpy(), r[0, :, :, :n], rtol=TOL_REL,
+                                   atol=TOL_ABS)
+        at += n
