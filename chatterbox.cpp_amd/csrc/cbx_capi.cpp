@@ -235,6 +235,11 @@ int cbx_sampler_create(cbx_sampler** out, int32_t device, int32_t max_vocab, int
     if (e == hipSuccess) e = hipMalloc(&s->d_probs, sizeof(float) * max_vocab);
     if (e == hipSuccess) e = hipMalloc(&s->d_redo, sizeof(int32_t) * cbx::kRedoWords);
     if (e == hipSuccess) e = hipMalloc(&s->d_redo_row, sizeof(int32_t) * 3);
+    // the head's split buffer, enough for every call of fewer than 16 rows
+    // that the mat-vec's LDS could hold (32 padded rows with CFG): such calls
+    // do not allocate
+    s->head_bytes = cbx::head_scratch_bytes(16, true, 2240);
+    if (e == hipSuccess) e = hipMalloc(&s->d_head, s->head_bytes);
     // the lists start empty; each redo pass leaves them empty again
     if (e == hipSuccess) e = hipMemset(s->d_redo, 0, sizeof(int32_t) * cbx::kRedoWords);
     if (e == hipSuccess) e = hipMemset(s->d_redo_row, 0, sizeof(int32_t) * 3);

@@ -8,7 +8,7 @@
 // little-endian word qh whose bit j is the fifth bit of element j, and the
 // nibbles as Q4_0's, w = (q - 16) d; Q8_0 blocks are d and 32 int8, w = q d).
 //
-// 16 rows and more run on the fp16 matrix cores in two launches:
+// 7 rows and more run on the fp16 matrix cores in two launches:
 //  * head_split: each activation row r is scaled by a power of two 2^s_r (its
 //    largest magnitude to [2^14, 2^15)) and written as two fp16 parts,
 //    x 2^s = hi + lo + e with |e| <= 2^-23 |x 2^s| + 2^-25 (hi and lo rounded
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == C
 }
 
 // ----------------------------------------------------------------- mat-vec
-// Fewer than 16 projected rows (a CFG pair is 2): no row tile to fill, so
+// Fewer than 7 projected rows (a CFG pair is 2): no row tile to fill, so
 // the weights are read once by plain FMAs.  The R rows of activations are
 // staged in LDS with each 32-element block padded to 33 words; LANES lanes
 // (16, or 32 / 64 for narrow outputs with long rows) take one vocab row, lane
@@ -734,11 +734,8 @@ hipError_t launch_gemv_r(const void* W, const float* bias, const float* hidden0,
     if (R <= 4)
         return launch_gemv<WT, 4>(W, bias, hidden0, hidden1, ld_hidden, out0, out1, ld_out, n_rows,
                                   n_vocab, n_embd, stream, gelu);
-    if (R <= 8)
-        return launch_gemv<WT, 8>(W, bias, hidden0, hidden1, ld_hidden, out0, out1, ld_out, n_rows,
-                                  n_vocab, n_embd, stream, gelu);
-    return launch_gemv<WT, 16>(W, bias, hidden0, hidden1, ld_hidden, out0, out1, ld_out, n_rows,
-                               n_vocab, n_embd, stream, gelu);
+    return launch_gemv<WT, 6>(W, bias, hidden0, hidden1, ld_hidden, out0, out1, ld_out, n_rows,
+                              n_vocab, n_embd, stream, gelu);
 }
 
 template <int WT, int NT>
@@ -813,9 +810,13 @@ hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const 
 
 }  // namespace
 
+// The mat-vec's work grows with its rows, the matrix cores' does not below 16,
+// and their two launches take 11 us: us per call at V = 6563, n_embd = 1024,
+// mat-vec / matrix cores, 3 rows 7.6 / 11.1, 5 10.4 / 11.2, 7 12.2 / 11.2, 12
+// 19.2 / 11.2 (Q8_0; the other formats within 0.2).
 bool head_uses_gemv(int32_t n_rows, bool cfg, int32_t n_embd) {
     const int R = cfg ? 2 * n_rows : n_rows;
-    return R < 16 && (size_t)R * gemv_row_words(n_embd) * 4 <= 65536;
+    return R < 7 && (size_t)R * gemv_row_words(n_embd) * 4 <= 65536;
 }
 
 size_t head_scratch_bytes(int32_t n_rows, bool cfg, int32_t n_embd) {
@@ -832,7 +833,6 @@ hipError_t launch_head(const void* W, int32_t wtype, const float* bias, const fl
 }
 
 int head_k_split(int32_t n_rows, int32_t n_vocab, int32_t n_embd) {
-    if (head_uses_gemv(n_rows, false, n_embd)) return 1;
     const int64_t wg = (int64_t)((n_vocab + 31) / 32) * ((n_rows + 15) / 16);  // one tile each
     const int nball = n_embd / 32;
     int kz = 1;
@@ -844,7 +844,7 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
                          const float* hidden1, int64_t ld_hidden, float* out0, float* out1,
                          int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                          void* scratch, hipStream_t stream, int kz, bool gelu_out) {
-    // fewer than 16 projected rows: the mat-vec (activations staged in LDS,
+    // fewer than 7 projected rows: the mat-vec (activations staged in LDS,
     // at most 64 KiB of them), else the split and the 16-row matrix-core tiles
     const bool cfg = hidden1 != nullptr;
     if (kz < 1 || (kz > 1 && (cfg || gelu_out || head_uses_gemv(n_rows, cfg, n_embd))))
@@ -889,7 +889,7 @@ hipError_t launch_head_presplit(const void* W, int32_t wtype, const float* bias,
                                 int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                                 const void* scratch, hipStream_t stream, int kz, bool gelu_out,
                                 void* out_split) {
-    if (!scratch || kz < 1 || head_uses_gemv(n_rows, false, n_embd) || (gelu_out && kz > 1) ||
+    if (!scratch || kz < 1 || (gelu_out && kz > 1) ||
         (out_split && (kz > 1 || n_vocab % 32 != 0)))
         return hipErrorInvalidValue;
     const int n_tiles = (n_rows + 15) / 16, R = 16 * n_tiles;

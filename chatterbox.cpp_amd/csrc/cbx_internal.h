@@ -118,7 +118,7 @@ hipError_t launch_decode_v1024x32(const KernelArgs& a, hipStream_t stream);
 // for r < n_rows, v < n_vocab, and the same from hidden1 into out1 in the same
 // launches when hidden1 is given.  `scratch` is device memory of at least
 // head_scratch_bytes(n_rows, hidden1 != NULL, n_embd) bytes (the activations
-// split for the matrix cores; 0 bytes, and NULL allowed, below 16 rows).
+// split for the matrix cores; 0 bytes, and NULL allowed, where head_uses_gemv).
 size_t head_scratch_bytes(int32_t n_rows, bool cfg, int32_t n_embd);
 // Bytes per block of 32 weights of a CBX_WTYPE_* (0 for an unknown type).
 inline int64_t wtype_block_bytes(int32_t wtype) {
@@ -130,15 +130,15 @@ inline int64_t wtype_block_bytes(int32_t wtype) {
         default: return 0;
     }
 }
-// Whether launch_head takes the mat-vec (fewer than 16 projected rows whose
+// Whether launch_head takes the mat-vec (fewer than 7 projected rows whose
 // activations fit its LDS) rather than the split and the matrix cores.
 bool head_uses_gemv(int32_t n_rows, bool cfg, int32_t n_embd);
 // launch_head with the products' K split over kz workgroups (one row set, the
 // matrix-core path): slab z of out0 (out0 + z * n_rows * ld_out) holds the
 // partial products of the z-th run of blocks, the bias in slab 0 only; the
-// caller adds the kz slabs.  head_k_split: the kz that launch would use
-// (1 for the mat-vec, else doubled up to 8 while the grid holds fewer than
-// 512 workgroups and each wave keeps 4 blocks).
+// caller adds the kz slabs.  head_k_split: the kz for the matrix cores
+// (doubled up to 8 while the grid holds fewer than 512 workgroups and each
+// wave keeps 4 blocks).
 // gelu_out: the T3 MLP's gelu (t3_gelu_f) applied to every output as it is
 // stored (no K split then).
 int head_k_split(int32_t n_rows, int32_t n_vocab, int32_t n_embd);
@@ -148,7 +148,7 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
                          void* scratch, hipStream_t stream, int kz, bool gelu_out);
 // The matrix-core products of n_rows rows already split into `scratch` by
 // their producer (cbx_split.h's layout, n_rows padded to whole 16-row tiles):
-// launch_head_k without its split launch (one row set; 16 rows and more).
+// launch_head_k without its split launch (one row set, any number of rows).
 // out_split set (no K split, n_vocab a multiple of 32): the outputs go there
 // split for the next product (rows of n_vocab) instead of to out0.
 hipError_t launch_head_presplit(const void* W, int32_t wtype, const float* bias, float* out0,

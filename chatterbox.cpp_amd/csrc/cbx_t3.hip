@@ -20,8 +20,8 @@
 //
 // The four matrix products of a layer have the speech_head's shape (rows of
 // n_in weights per output, F16 / Q4_0 / Q5_0 / Q8_0): they run on the head's
-// kernels (fp16 matrix cores on split activations from 16 rows, a mat-vec
-// below).  From 16 rows the layer norms write the split activations of the
+// kernels (fp16 matrix cores on split activations from 4 rows, a mat-vec
+// below).  From 4 rows the layer norms write the split activations of the
 // products they feed themselves, and the two products the residual adds
 // take a K split over workgroups when their grid is narrow, their slabs
 // added by the norm that follows; gelu is applied as the mlp c_fc product
@@ -720,12 +720,27 @@ bool t3_attn_wide(int32_t n_rows, int32_t n_head) { return (int64_t)n_rows * n_h
 // c_fc the second (c_fc reads the first as it writes), then, where the rows are
 // many (head_uses_tiles), the largest matrix unpacked for its product.
 
+// Streams on the matrix cores, every product's input written split by its
+// producer; fewer run the mat-vecs on plain rows.  us per step of the Turbo
+// shape at position 256, mat-vecs / matrix cores: Q4_0 4 streams 1146 / 1012, 6
+// 1381 / 1052, 8 1497 / 1050, 15 2128 / 1115; Q8_0 6 1406 / 1107.  (3 streams,
+// 1153 / 982, stay: their rows are bit for bit those of one or two.)
+static bool t3_matrix(int32_t n_rows, int32_t n_embd) {
+    return n_rows >= 4 || !head_uses_gemv(n_rows, false, n_embd);
+}
+
+// Bytes of one split buffer of the widest input (also where the mat-vecs'
+// LDS cannot hold rows of 4 n_embd).
+static size_t t3_split_bytes(int32_t n_rows, int32_t n_embd) {
+    if (!t3_matrix(n_rows, n_embd) && head_uses_gemv(n_rows, false, 4 * n_embd)) return 0;
+    return (split_bytes((n_rows + 15) / 16 * 16, 4 * n_embd) + 255) / 256 * 256;
+}
+
 size_t t3_workspace_bytes(int32_t n_rows, int32_t n_embd) {
     const size_t row = (size_t)n_rows * n_embd * 4;
     const size_t body = (3 + kMaxKSplit) * row + 3 * row + 4 * row +
                         ((size_t)n_rows * 4 + 255) / 256 * 256;
-    const size_t sp = (head_scratch_bytes(n_rows, false, 4 * n_embd) + 255) / 256 * 256;
-    return body + 2 * sp + max(tile_scratch_bytes(n_rows, 4 * n_embd, n_embd),
+    return body + 2 * t3_split_bytes(n_rows, n_embd) + max(tile_scratch_bytes(n_rows, 4 * n_embd, n_embd),
                                tile_scratch_bytes(n_rows, n_embd, 4 * n_embd));
 }
 
@@ -747,10 +762,8 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     int32_t* act = reinterpret_cast<int32_t*>(f + 4 * row);
     const bool wide = !prefill && t3_attn_wide(n_rows, m.n_head);
     void* split = reinterpret_cast<char*>(act) + ((size_t)n_rows * 4 + 255) / 256 * 256;
-    void* split2 = static_cast<char*>(split) +
-                   (head_scratch_bytes(n_rows, false, 4 * n) + 255) / 256 * 256;
-    void* unpacked = static_cast<char*>(split2) +
-                     (head_scratch_bytes(n_rows, false, 4 * n) + 255) / 256 * 256;
+    void* split2 = static_cast<char*>(split) + t3_split_bytes(n_rows, n);
+    void* unpacked = static_cast<char*>(split2) + t3_split_bytes(n_rows, n);
 
     NormArgs na{};
     na.n_embd = n;
@@ -771,10 +784,9 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     na.g = m.layers[0].ln_1_g;
     na.b = m.layers[0].ln_1_b;
     na.out = u;
-    // 16 streams and more (the matrix-core path): every product's input is
-    // written split by its producer (the norms, the attention, c_fc); below,
-    // plain rows for the mat-vec
-    const bool mc = !head_uses_gemv(n_rows, false, n);
+    // on the matrix cores every product's input is written split by its
+    // producer (the norms, the attention, c_fc); else plain rows
+    const bool mc = t3_matrix(n_rows, n);
     uint32_t* const sparts = static_cast<uint32_t*>(split);
     float* const sinv = reinterpret_cast<float*>(static_cast<char*>(split) +
                                                  split_inv_offset(16 * ((n_rows + 15) / 16), n));
@@ -799,8 +811,9 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     aa.scale = 0.125f;  // 1 / sqrt(64)
     const size_t lds = t3_attn_lds(c.n_ctx);
 
-    const int kz_a = min(head_k_split(n_rows, n, n), kMaxKSplit);
-    const int kz_f = min(head_k_split(n_rows, n, 4 * n), kMaxKSplit);
+    const int kz_a = mc ? min(head_k_split(n_rows, n, n), kMaxKSplit) : 1;
+    const int kz_f = mc || !head_uses_gemv(n_rows, false, 4 * n)
+                         ? min(head_k_split(n_rows, n, 4 * n), kMaxKSplit) : 1;
     // one or two streams: the residual adds and norms between the layer's
     // products run inside the mat-vec that consumes them (c_fc, and the next
     // layer's c_attn), the residual rows alternating between x and y's

@@ -187,3 +187,32 @@ def test_many_rows_products(small, wtype, lens):
                 assert np.allclose(c[b, :, :, :n].cpu().numpy(), r[0, :, :, :n], rtol=TOL_REL,
                                    atol=TOL_ABS)
         at += n
+
+
+@pytest.mark.parametrize("n_streams", [3, 4, 7, 15, 16, 17])
+@pytest.mark.parametrize("wtype", [O.WTYPE_F16, O.WTYPE_Q4_0, O.WTYPE_Q5_0, O.WTYPE_Q8_0])
+def test_step_at_the_row_edges(small, wtype, n_streams):
+    """Decode steps either side of 4 streams (mat-vecs below, matrix cores from
+    there) and of a whole row tile, one stream sitting the second step out."""
+    torch, s = small[:2]
+    dm, rm = model(torch, pkg.load(), wtype)
+    rng = np.random.default_rng(100 * wtype + n_streams)
+    k = torch.full((n_streams, L_, H, 8, 64), float("nan"), device="cuda")
+    v = k.clone()
+    pos = torch.zeros(n_streams, dtype=torch.int32, device="cuda")
+    hid = torch.full((n_streams, N), 7.0, device="cuda")
+    kr, vr = T3.new_cache(n_streams, L_, H, 8)
+    at = np.zeros(n_streams, np.int64)
+    for t in range(3):
+        toks = rng.integers(0, V, n_streams).astype(np.int32)
+        state = np.zeros(n_streams, np.int32)
+        state[n_streams // 2] = t == 1
+        print(f"[gpu-case] step wtype={wtype} streams={n_streams} t={t}", flush=True)
+        s.t3_step(dm, pos, k, v, hid, tokens=torch.from_numpy(toks).cuda(),
+                  state=torch.from_numpy(state).cuda())
+        torch.cuda.synchronize()
+        got = hid.cpu().numpy()
+        want = T3.step(rm, toks, at, kr, vr, active=state == 0)
+        err = np.abs(got - want)
+        assert np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), f"step {t}: {err.max():.3g}"
+        assert np.array_equal(pos.cpu().numpy(), at)
