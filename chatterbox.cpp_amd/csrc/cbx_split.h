@@ -150,8 +150,8 @@ __host__ __device__ inline int64_t split_inv_index(int T, int m, int nball, int 
 // The largest magnitude over the 4 consecutive lanes (lane & ~3 .. + 3) that
 // hold one block's 4 groups.
 __device__ __forceinline__ float split_block_max4(float mx) {
-    mx = fmaxf(mx, __shfl_xor(mx, 1));
-    return fmaxf(mx, __shfl_xor(mx, 2));
+    mx = fmaxf(mx, dpp16<0xB1>(mx));
+    return fmaxf(mx, dpp16<0x4E>(mx));
 }
 
 }  // namespace cbx

@@ -36,6 +36,7 @@
 
 #include "cbx_internal.h"
 #include "cbx_split.h"
+#include "cbx_weights.h"
 #include "../../include/cbx_t3.h"
 
 namespace cbx {
@@ -72,36 +73,19 @@ struct NormArgs {
     int32_t advance;       // last norm of the step: positions[r] += 1
 };
 
-// One row per workgroup: the embedding or the residual add, then the layer
-// norm.  Inactive rows (streams that take no step) keep x and write zeros.
-// The next product's split activations for row r from its values in LDS: 8
-// consecutive values per group, groups tid, tid + 256, ..., each block's
-// scale from the largest magnitude of its 4 groups (4 consecutive threads).
-__device__ __forceinline__ void norm_split(const NormArgs& a, int r, const float* row_s) {
-    const int n = a.n_embd, tid = threadIdx.x, nball = n / 32;
-    for (int j0 = 0; j0 < n / 8; j0 += kNormThreads) {  // whole waves in or out
-        const int j = j0 + tid;
-        if (j0 + (tid & ~63) >= n / 8) break;
-        float v[8];
-        float mx = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            v[i] = j < n / 8 ? row_s[8 * j + i] : 0.0f;
-            mx = fmaxf(mx, fabsf(v[i]));
-        }
-        mx = split_block_max4(mx);
-        if (j >= n / 8) continue;
-        float sc, sinv;
-        split_scale(mx, sc, sinv);
-        split_store(a.parts, r >> 4, r & 15, nball, j, v, sc);
-        if ((j & 3) == 0) a.inv[split_inv_index(r >> 4, r & 15, nball, j >> 2)] = sinv;
-    }
+// Whether row r takes this step (embedding mode; stored for the norms after).
+__device__ __forceinline__ bool norm_active(const NormArgs& a, int r, int pos, int tok) {
+    const int slot = a.slots ? a.slots[r] : r;
+    return (!a.state || a.state[r] == CBX_DECODE_RUNNING) && pos >= 0 && pos < a.n_ctx &&
+           pos < a.n_pos && (a.inputs || (tok >= 0 && tok < a.n_vocab)) &&
+           (!a.slots || (slot >= 0 && slot < a.n_slots));
 }
 
+// One row per workgroup: the embedding or the residual add, then the layer
+// norm.  Inactive rows (streams that take no step) keep x and write zeros.
 template <int EPT>
 __global__ __launch_bounds__(kNormThreads) void t3_norm(NormArgs a) {
     __shared__ float red[8];
-    __shared__ float row_s[EPT * kNormThreads];
     int ph = 0;
     const int r = blockIdx.x, tid = threadIdx.x;
     const int n = a.n_embd;
@@ -112,21 +96,13 @@ __global__ __launch_bounds__(kNormThreads) void t3_norm(NormArgs a) {
     if (a.emb || a.inputs) {
         const int pos = a.positions[r];
         const int tok = a.tokens ? a.tokens[r] : 0;
-        const int slot = a.slots ? a.slots[r] : r;
-        active = (!a.state || a.state[r] == CBX_DECODE_RUNNING) && pos >= 0 && pos < a.n_ctx &&
-                 pos < a.n_pos && (a.inputs || (tok >= 0 && tok < a.n_vocab)) &&
-                 (!a.slots || (slot >= 0 && slot < a.n_slots));
+        active = norm_active(a, r, pos, tok);
         if (tid == 0) a.act[r] = active ? 1 : 0;
         if (!active) {
 #pragma unroll
             for (int j = 0; j < EPT; ++j) {
                 xr[j * kNormThreads + tid] = 0.0f;
-                row_s[j * kNormThreads + tid] = 0.0f;
-                if (!a.parts) orow[j * kNormThreads + tid] = 0.0f;
-            }
-            if (a.parts) {
-                __syncthreads();
-                norm_split(a, r, row_s);
+                orow[j * kNormThreads + tid] = 0.0f;
             }
             return;
         }
@@ -145,14 +121,7 @@ __global__ __launch_bounds__(kNormThreads) void t3_norm(NormArgs a) {
         active = a.act[r] != 0;
         if (!active) {
 #pragma unroll
-            for (int j = 0; j < EPT; ++j) {
-                row_s[j * kNormThreads + tid] = 0.0f;
-                if (!a.parts) orow[j * kNormThreads + tid] = 0.0f;
-            }
-            if (a.parts) {
-                __syncthreads();
-                norm_split(a, r, row_s);
-            }
+            for (int j = 0; j < EPT; ++j) orow[j * kNormThreads + tid] = 0.0f;
             return;
         }
         // the product's slabs (all loads issued first), added in slab order,
@@ -193,18 +162,125 @@ __global__ __launch_bounds__(kNormThreads) void t3_norm(NormArgs a) {
     for (int j = 0; j < EPT; ++j) {
         const int i = j * kNormThreads + tid;
         xr[i] = xv[j];
-        const float o =
-            __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(xv[j], mean), scale), a.g[i]), a.b[i]);
-        if (a.parts)
-            row_s[i] = o;
-        else
-            orow[i] = o;
-    }
-    if (a.parts) {
-        __syncthreads();  // row_s complete
-        norm_split(a, r, row_s);
+        orow[i] = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(xv[j], mean), scale), a.g[i]), a.b[i]);
     }
     if (a.advance && tid == 0) a.positions[r] += 1;
+}
+
+// The same with the norm's rows written split for the matrix cores (a.parts):
+// thread j holds values 8j .. 8j + 7 of the row, a group of the split, so the
+// loads are 16 bytes a lane and the values go from the sums to the split in
+// registers (256 threads of every 256th value each passed them through the
+// LDS and left half the threads without a group at 1024).
+// us per step or pass at n_embd 1024 (48 of these), 256 threads -> here: 64
+// streams 1605 -> 1517, 6 streams Q8_0 1115 -> 1025, one prompt of 251 rows 1815
+// -> 1743, 64 prompts of 129-383 rows 31710 -> 31650.
+constexpr int kNormSplitMax = 512;  // n_embd 4096
+template <int NY>
+__global__ __launch_bounds__(kNormSplitMax) void t3_norm_split(NormArgs a) {
+    __shared__ float red[2][kNormSplitMax / 64];
+    const int r = blockIdx.x, j = threadIdx.x, n = a.n_embd, nw = (int)blockDim.x / 64;
+    const bool in = 8 * j < n;  // n_embd 256, 768: the last wave's rest
+    const int k = in ? 8 * j : 0;
+    float* const xr = a.x + (int64_t)r * n + k;
+    const auto load8 = [](const float* p, float (&v)[8]) {
+        const f4 u = *reinterpret_cast<const f4*>(p), w = *reinterpret_cast<const f4*>(p + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = u[i];
+            v[4 + i] = w[i];
+        }
+    };
+    const auto store8 = [](float* p, const float (&v)[8]) {
+        *reinterpret_cast<f4*>(p) = f4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f4*>(p + 4) = f4{v[4], v[5], v[6], v[7]};
+    };
+    float xv[8], gv[8], bv[8];
+    bool active;
+    if constexpr (NY == 0) {  // the embedding or the input row
+        const int pos = a.positions[r];
+        const int tok = a.tokens ? a.tokens[r] : 0;
+        active = norm_active(a, r, pos, tok);
+        if (j == 0) a.act[r] = active ? 1 : 0;
+        if (active && a.inputs) {
+            const float* const p = a.inputs + (int64_t)r * n + k;  // of any alignment
+#pragma unroll
+            for (int i = 0; i < 8; ++i) xv[i] = p[i];
+        } else if (active) {
+            const float* const e = a.emb + (int64_t)tok * n + k;
+            const float* const p = a.wpe + (int64_t)pos * n + k;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) xv[i] = __fadd_rn(e[i], p[i]);
+        }
+    } else {
+        // the product's slabs, added in slab order, then the residual
+        // (main.cpp:551, :559); loaded beside the flag
+        float ys[NY][8];
+        active = a.act[r] != 0;
+        load8(xr, xv);
+#pragma unroll
+        for (int z = 0; z < NY; ++z) load8(a.y + (int64_t)z * a.ystride + (int64_t)r * n + k, ys[z]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            float c = ys[0][i];
+#pragma unroll
+            for (int z = 1; z < NY; ++z) c = __fadd_rn(c, ys[z][i]);
+            xv[i] = __fadd_rn(c, xv[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        gv[i] = a.g[k + i];
+        bv[i] = a.b[k + i];
+    }
+    if (!active) {
+        if (!in) return;
+        const float zero[8] = {};
+        if (NY == 0) store8(xr, zero);
+        split_store(a.parts, r >> 4, r & 15, n / 32, j, zero, 1.0f);
+        if ((j & 3) == 0) a.inv[split_inv_index(r >> 4, r & 15, n / 32, j >> 2)] = 1.0f;
+        return;
+    }
+    // a wave's sum as block_sum256's, the waves' in order
+    const auto block_sum = [&](float v, float* h) {
+        v = sum16_dpp(in ? v : 0.0f);
+        const auto lane_v = [&](int l) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+        };
+        const float w = __fadd_rn(__fadd_rn(lane_v(0), lane_v(16)), __fadd_rn(lane_v(32), lane_v(48)));
+        if (nw == 1) return w;
+        if ((j & 63) == 0) h[j >> 6] = w;
+        __syncthreads();
+        float s = h[0];
+        for (int i = 1; i < nw; ++i) s = __fadd_rn(s, h[i]);
+        return s;
+    };
+    const auto sum8 = [](const float (&v)[8]) {
+        return __fadd_rn(__fadd_rn(__fadd_rn(v[0], v[1]), __fadd_rn(v[2], v[3])),
+                         __fadd_rn(__fadd_rn(v[4], v[5]), __fadd_rn(v[6], v[7])));
+    };
+    const float mean = __fdiv_rn(block_sum(sum8(xv), red[0]), (float)n);
+    float d[8], q[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        d[i] = __fsub_rn(xv[i], mean);
+        q[i] = __fmul_rn(d[i], d[i]);
+    }
+    const float var = __fdiv_rn(block_sum(sum8(q), red[1]), (float)n);
+    const float scale = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(var, a.eps)));
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        d[i] = __fadd_rn(__fmul_rn(__fmul_rn(d[i], scale), gv[i]), bv[i]);
+        mx = fmaxf(mx, fabsf(d[i]));
+    }
+    mx = split_block_max4(mx);
+    if (!in) return;
+    store8(xr, xv);
+    float sc, sinv;
+    split_scale(mx, sc, sinv);
+    split_store(a.parts, r >> 4, r & 15, n / 32, j, d, sc);
+    if ((j & 3) == 0) a.inv[split_inv_index(r >> 4, r & 15, n / 32, j >> 2)] = sinv;
 }
 
 struct AttnArgs {
@@ -253,9 +329,8 @@ __device__ __forceinline__ void attn_store(const AttnArgs& a, int r, int h, int 
     if (k == 0) a.inv[split_inv_index(T, m, nball, kb)] = sinv;
 }
 
-typedef float mf4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ mf4 mfma_f32(float x, float y, const mf4& acc) {
+__device__ __forceinline__ f4 mfma_f32(float x, float y, const f4& acc) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0);
 }
 
@@ -264,10 +339,10 @@ __device__ __forceinline__ mf4 mfma_f32(float x, float y, const mf4& acc) {
 // n_rows): to out, or split as attn_store does (block 2h + c / 8, its largest
 // magnitude over 8 lanes).
 __device__ __forceinline__ void attn_store4(const AttnArgs& a, int n_rows, int r, int h, int c,
-                                            const mf4& o) {
+                                            const f4& o) {
     if (!a.parts) {
         if (r < n_rows)
-            *reinterpret_cast<mf4*>(a.out + (int64_t)r * a.n_head * kHeadDim + h * kHeadDim + 4 * c) = o;
+            *reinterpret_cast<f4*>(a.out + (int64_t)r * a.n_head * kHeadDim + h * kHeadDim + 4 * c) = o;
         return;
     }
     float mx = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fmaxf(fabsf(o[2]), fabsf(o[3])));
@@ -486,13 +561,13 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
     const int rc = min(r0 + c, n_rows - 1);
     const bool real = r0 + c < n_rows && a.act[rc] != 0;
     const int pos = a.positions[rc], slot = a.slots[rc];
-    mf4 q[4], o[4];
+    f4 q[4], o[4];
     {
         const float* const qr = a.qkv + (int64_t)rc * 3 * n + h * kHeadDim + 4 * g;
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
-            q[cc] = *reinterpret_cast<const mf4*>(qr + 16 * cc);
-            o[cc] = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+            q[cc] = *reinterpret_cast<const f4*>(qr + 16 * cc);
+            o[cc] = f4{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
     float m = -INFINITY, s = 0.0f;
@@ -521,23 +596,23 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
         const float* const vc = a.vc + base;
         for (int j0 = KS == 1 ? 0 : 16 * KT * w; j0 <= last; j0 += 16 * KT * KS) {
             // keys past the last read the last one's row, at weight 0
-            mf4 kk[KT][4], vv[KT][4], p[KT];
+            f4 kk[KT][4], vv[KT][4], p[KT];
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) {
                 const float* const kr =
                     kc + (int64_t)min(j0 + 16 * kt + c, last) * kHeadDim + 4 * g;
 #pragma unroll
                 for (int cc = 0; cc < 4; ++cc)
-                    kk[kt][cc] = *reinterpret_cast<const mf4*>(kr + 16 * cc);
+                    kk[kt][cc] = *reinterpret_cast<const f4*>(kr + 16 * cc);
             }
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    vv[kt][v] = *reinterpret_cast<const mf4*>(
+                    vv[kt][v] = *reinterpret_cast<const f4*>(
                         vc + (int64_t)min(j0 + 16 * kt + 4 * g + v, last) * kHeadDim + 4 * c);
 #pragma unroll
-            for (int kt = 0; kt < KT; ++kt) p[kt] = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int kt = 0; kt < KT; ++kt) p[kt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int cc = 0; cc < 4; ++cc)
 #pragma unroll
@@ -600,7 +675,7 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
                     const int li = __builtin_amdgcn_readlane(lim, i);
 #pragma unroll
                     for (int dt = 0; dt < 4; ++dt) {
-                        mf4 add = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+                        f4 add = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -623,17 +698,17 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
         for (int v = 0; v < 4; ++v) {
             const float sv = __shfl(s, 4 * g + v);
             const bool on = __shfl((int)real, 4 * g + v) != 0;
-            mf4 x;
+            f4 x;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) x[dt] = on ? __fdiv_rn(o[dt][v], sv) : 0.0f;
             attn_store4(a, n_rows, r0 + 4 * g + v, h, c, x);
         }
     } else {
         // wave w joins the four waves' rows 4 g + w
-        __shared__ mf4 os[KS][4][64];
+        __shared__ f4 os[KS][4][64];
         __shared__ float ms[KS][16], ss[KS][16];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) os[w][v][lane] = mf4{o[0][v], o[1][v], o[2][v], o[3][v]};
+        for (int v = 0; v < 4; ++v) os[w][v][lane] = f4{o[0][v], o[1][v], o[2][v], o[3][v]};
         if (g == 0) {
             ms[w][c] = m;
             ss[w][c] = s;
@@ -644,12 +719,12 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
 #pragma unroll
         for (int x = 1; x < KS; ++x) M = fmaxf(M, ms[x][i]);
         float st = 0.0f;
-        mf4 at = mf4{0.0f, 0.0f, 0.0f, 0.0f};
+        f4 at = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int x = 0; x < KS; ++x) {
             const float f = ms[x][i] == -INFINITY ? 0.0f : expf(__fsub_rn(ms[x][i], M));
             st = __fadd_rn(st, __fmul_rn(ss[x][i], f));
-            const mf4 ov = os[x][w][lane];
+            const f4 ov = os[x][w][lane];
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) at[dt] = __fadd_rn(at[dt], __fmul_rn(ov[dt], f));
         }
@@ -682,7 +757,24 @@ hipError_t launch_attn_tile(const AttnArgs& a, int n_rows, hipStream_t st) {
     return hipGetLastError();
 }
 
+template <int NY>
+hipError_t launch_norm_split(const NormArgs& a, int n_rows, hipStream_t st) {
+    hipLaunchKernelGGL(t3_norm_split<NY>, dim3((unsigned)n_rows),
+                       dim3((unsigned)((a.n_embd / 8 + 63) / 64 * 64)), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_norm(const NormArgs& a, int n_rows, hipStream_t st) {
+    if (a.parts) {  // slabs: none (the embedding) or a power of two
+        switch (a.y ? a.ny : 0) {
+            case 0: return launch_norm_split<0>(a, n_rows, st);
+            case 1: return launch_norm_split<1>(a, n_rows, st);
+            case 2: return launch_norm_split<2>(a, n_rows, st);
+            case 4: return launch_norm_split<4>(a, n_rows, st);
+            case 8: return launch_norm_split<8>(a, n_rows, st);
+            default: return hipErrorInvalidValue;
+        }
+    }
     switch (a.n_embd / kNormThreads) {
         case 1: return launch_norm_ept<1>(a, n_rows, st);
         case 2: return launch_norm_ept<2>(a, n_rows, st);

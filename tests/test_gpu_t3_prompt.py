@@ -33,17 +33,17 @@ def small():
     s.close()
 
 
-def model(torch, mod, wtype):
+def model(torch, mod, wtype, N=N, H=H, sd=0.08):
     rng = np.random.default_rng(0x9A11)
     t = lambda a: torch.from_numpy(a).cuda()
     vec = lambda k, base=0.0, sd=0.1: (base + rng.standard_normal(k) * sd).astype(np.float32)
     dev, ref = [], []
-    for _ in range(L_):
+    for _ in range(L_ if N == 256 else 1):
         d, r = {}, {}
         for key, o, i in (("attn_w", 3, 1), ("attn_proj_w", 1, 1), ("fc_w", 4, 1),
                           ("fc_proj_w", 1, 4)):
             # large enough that some scores stand out: the running max grows
-            w = (rng.standard_normal((o * N, i * N)) * 0.08).astype(np.float32)
+            w = (rng.standard_normal((o * N, i * N)) * sd).astype(np.float32)
             blocks = O.quantize(w, wtype)
             d[key], r[key] = t(blocks.reshape(-1)), O.dequantize(blocks, wtype, i * N)
         for key, k, base in (("ln_1_g", N, 1.0), ("ln_1_b", N, 0.0), ("attn_b", 3 * N, 0.0),
@@ -216,3 +216,38 @@ def test_step_at_the_row_edges(small, wtype, n_streams):
         err = np.abs(got - want)
         assert np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), f"step {t}: {err.max():.3g}"
         assert np.array_equal(pos.cpu().numpy(), at)
+
+
+@pytest.mark.parametrize("n_head", [4, 8, 12, 24])
+def test_split_norm_widths(small, n_head):
+    """The split norm where a row fills part of a wave (n_embd 256), one, one and
+    a half and three waves: two steps of 5 streams, one sitting the second out,
+    and 19 prompt rows."""
+    torch, s = small[:2]
+    dm, rm = model(torch, pkg.load(), O.WTYPE_Q8_0, 64 * n_head, n_head, sd=0.02)
+    rng = np.random.default_rng(n_head)
+    n = 64 * n_head
+    layers = L_ if n == 256 else 1
+    k = torch.full((5, layers, n_head, 24, 64), float("nan"), device="cuda")
+    v = k.clone()
+    kr, vr = T3.new_cache(5, layers, n_head, 24)
+    x = (rng.standard_normal((19, n)) * 0.7).astype(np.float32)
+    hid = torch.empty((19, n), device="cuda")
+    print(f"[gpu-case] split norm n_embd={n}", flush=True)
+    s.t3_prefill(dm, torch.zeros(19, dtype=torch.int32, device="cuda"),
+                 torch.arange(19, dtype=torch.int32, device="cuda"), k, v, hid,
+                 inputs=torch.from_numpy(x).cuda())
+    torch.cuda.synchronize()
+    want = T3.prefill(rm, x, kr, vr, 0, 0)
+    assert np.all(np.abs(hid.cpu().numpy() - want) <= TOL_ABS + TOL_REL * np.abs(want))
+    at = np.array([19, 0, 0, 0, 0], np.int64)
+    pos = torch.from_numpy(at.astype(np.int32)).cuda()
+    hid = torch.empty((5, n), device="cuda")
+    for t in range(2):
+        toks = rng.integers(0, V, 5).astype(np.int32)
+        state = np.array([0, 0, t, 0, 0], np.int32)
+        s.t3_step(dm, pos, k, v, hid, tokens=torch.from_numpy(toks).cuda(),
+                  state=torch.from_numpy(state).cuda())
+        torch.cuda.synchronize()
+        want = T3.step(rm, toks, at, kr, vr, active=state == 0)
+        assert np.all(np.abs(hid.cpu().numpy() - want) <= TOL_ABS + TOL_REL * np.abs(want))
