@@ -34,6 +34,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "cbx_internal.h"
 #include "cbx_split.h"
 #include "cbx_weights.h"
@@ -140,13 +142,14 @@ constexpr int RING = 2;
 // applied when gelu_out, are written as the next product's split activations
 // (rows of n_vocab values: this workgroup's 32 outputs are block blockIdx.x
 // of each of its rows) instead of fp32 rows.
-template <int WT, int NT>
+// KV: a q|k|v product, its k and v stored in the caches (kv_place).
+template <int WT, int NT, bool KV>
 __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == CBX_WTYPE_Q4_0 ? 4 : 1))) void head_mfma(const void* W, const float* bias,
                                                      const uint32_t* parts, const float* inv,
                                                      int n_tiles, float* out0, float* out1,
                                                      int64_t ld_out, int n_rows, int n_vocab,
                                                      int n_embd, int64_t zstride, int gelu_out,
-                                                     uint32_t* out_parts, float* out_inv) {
+                                                     uint32_t* out_parts, float* out_inv, KvOut kv) {
     constexpr int BB = block_bytes<WT>();
     // Weights are staged per wave in chunks of CB blocks: for each of the 32
     // vocab rows the chunk's CB * BB bytes are contiguous, so whole-row dword
@@ -363,6 +366,14 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == C
                 float* orow = o + (int64_t)rr * ld_out;
                 const float xa = __fadd_rn(acc0[t][i], ba);
                 const float xb = __fadd_rn(acc1[t][i], bb);
+                if (KV && 3 * v0 >= n_vocab) {  // whole heads: va and vb in one
+                    float* const p = kv_place(kv, rr, va);
+                    if (p) {
+                        p[0] = xa;
+                        p[16] = xb;
+                    }
+                    continue;
+                }
                 if (va < n_vocab) orow[va] = gelu_out ? t3_gelu_f(xa) : xa;
                 if (vb < n_vocab) orow[vb] = gelu_out ? t3_gelu_f(xb) : xb;
             }
@@ -743,12 +754,17 @@ hipError_t launch_mfma(const void* W, const float* bias, const uint32_t* parts, 
                        int n_tiles, float* out0, float* out1, int64_t ld_out, int n_rows,
                        int n_vocab, int n_embd, hipStream_t stream, int kz = 1,
                        int gelu_out = 0, uint32_t* out_parts = nullptr,
-                       float* out_inv = nullptr) {
+                       float* out_inv = nullptr, const KvOut& kv = KvOut{}) {
     const dim3 grid((unsigned)((n_vocab + 31) / 32), (unsigned)((n_tiles + NT - 1) / NT),
                     (unsigned)kz);
-    hipLaunchKernelGGL((head_mfma<WT, NT>), grid, dim3(64 * KS), 0, stream, W, bias, parts, inv,
-                       n_tiles, out0, out1, ld_out, n_rows, n_vocab, n_embd,
-                       (int64_t)n_rows * ld_out, gelu_out, out_parts, out_inv);
+    if (kv.kc)
+        hipLaunchKernelGGL((head_mfma<WT, NT, true>), grid, dim3(64 * KS), 0, stream, W, bias,
+                           parts, inv, n_tiles, out0, out1, ld_out, n_rows, n_vocab, n_embd,
+                           (int64_t)n_rows * ld_out, 0, nullptr, nullptr, kv);
+    else
+        hipLaunchKernelGGL((head_mfma<WT, NT, false>), grid, dim3(64 * KS), 0, stream, W, bias,
+                           parts, inv, n_tiles, out0, out1, ld_out, n_rows, n_vocab, n_embd,
+                           (int64_t)n_rows * ld_out, gelu_out, out_parts, out_inv, kv);
     return hipGetLastError();
 }
 
@@ -761,50 +777,28 @@ hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const 
                          const float* inv, int n_tiles, float* out0, float* out1, int64_t ld_out,
                          int32_t n_rows, int32_t n_vocab, int32_t n_embd, hipStream_t stream,
                          int kz, int gelu_out, uint32_t* out_parts = nullptr,
-                         float* out_inv = nullptr) {
-    if ((int64_t)((n_vocab + 31) / 32) * ((n_tiles + 1) / 2) < 512 || kz > 1 || gelu_out ||
-        out_parts) {
-        switch (wtype) {
-            case CBX_WTYPE_F16:
-                return launch_mfma<CBX_WTYPE_F16, 1>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                     ld_out, n_rows, n_vocab, n_embd, stream, kz,
-                                                     gelu_out, out_parts, out_inv);
-            case CBX_WTYPE_Q4_0:
-                return launch_mfma<CBX_WTYPE_Q4_0, 1>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                      ld_out, n_rows, n_vocab, n_embd, stream, kz,
-                                                     gelu_out, out_parts, out_inv);
-            case CBX_WTYPE_Q5_0:
-                return launch_mfma<CBX_WTYPE_Q5_0, 1>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                      ld_out, n_rows, n_vocab, n_embd, stream, kz,
-                                                      gelu_out, out_parts, out_inv);
-            case CBX_WTYPE_Q8_0:
-                return launch_mfma<CBX_WTYPE_Q8_0, 1>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                      ld_out, n_rows, n_vocab, n_embd, stream, kz,
-                                                     gelu_out, out_parts, out_inv);
-            default:
-                return hipErrorInvalidValue;
-        }
-    }
+                         float* out_inv = nullptr, const KvOut& kv = KvOut{}) {
+    const bool one = (int64_t)((n_vocab + 31) / 32) * ((n_tiles + 1) / 2) < 512 || kz > 1 ||
+                     gelu_out || out_parts;
     const bool two = wtype == CBX_WTYPE_Q4_0 || wtype == CBX_WTYPE_Q5_0 || n_tiles <= 2;
+    auto run = [&](auto wt) {
+        constexpr int WT = decltype(wt)::value;
+        auto go = [&](auto nt) {
+            return launch_mfma<WT, decltype(nt)::value>(W, bias, parts, inv, n_tiles, out0, out1,
+                                                        ld_out, n_rows, n_vocab, n_embd, stream,
+                                                        kz, gelu_out, out_parts, out_inv, kv);
+        };
+        if (one) return go(std::integral_constant<int, 1>{});
+        if constexpr (WT == CBX_WTYPE_F16 || WT == CBX_WTYPE_Q8_0)
+            if (!two) return go(std::integral_constant<int, 4>{});
+        return go(std::integral_constant<int, 2>{});
+    };
     switch (wtype) {
-        case CBX_WTYPE_F16:
-            return two ? launch_mfma<CBX_WTYPE_F16, 2>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                       ld_out, n_rows, n_vocab, n_embd, stream)
-                       : launch_mfma<CBX_WTYPE_F16, 4>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                       ld_out, n_rows, n_vocab, n_embd, stream);
-        case CBX_WTYPE_Q4_0:
-            return launch_mfma<CBX_WTYPE_Q4_0, 2>(W, bias, parts, inv, n_tiles, out0, out1, ld_out,
-                                                  n_rows, n_vocab, n_embd, stream);
-        case CBX_WTYPE_Q5_0:
-            return launch_mfma<CBX_WTYPE_Q5_0, 2>(W, bias, parts, inv, n_tiles, out0, out1, ld_out,
-                                                  n_rows, n_vocab, n_embd, stream);
-        case CBX_WTYPE_Q8_0:
-            return two ? launch_mfma<CBX_WTYPE_Q8_0, 2>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                        ld_out, n_rows, n_vocab, n_embd, stream)
-                       : launch_mfma<CBX_WTYPE_Q8_0, 4>(W, bias, parts, inv, n_tiles, out0, out1,
-                                                        ld_out, n_rows, n_vocab, n_embd, stream);
-        default:
-            return hipErrorInvalidValue;
+        case CBX_WTYPE_F16: return run(std::integral_constant<int, CBX_WTYPE_F16>{});
+        case CBX_WTYPE_Q4_0: return run(std::integral_constant<int, CBX_WTYPE_Q4_0>{});
+        case CBX_WTYPE_Q5_0: return run(std::integral_constant<int, CBX_WTYPE_Q5_0>{});
+        case CBX_WTYPE_Q8_0: return run(std::integral_constant<int, CBX_WTYPE_Q8_0>{});
+        default: return hipErrorInvalidValue;
     }
 }
 
@@ -888,9 +882,10 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
 hipError_t launch_head_presplit(const void* W, int32_t wtype, const float* bias, float* out0,
                                 int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                                 const void* scratch, hipStream_t stream, int kz, bool gelu_out,
-                                void* out_split) {
+                                void* out_split, const KvOut& kv) {
     if (!scratch || kz < 1 || (gelu_out && kz > 1) ||
-        (out_split && (kz > 1 || n_vocab % 32 != 0)))
+        (out_split && (kz > 1 || n_vocab % 32 != 0)) ||
+        (kv.kc && (out_split || gelu_out || kz > 1 || n_vocab != 3 * 64 * kv.n_head)))
         return hipErrorInvalidValue;
     const int n_tiles = (n_rows + 15) / 16, R = 16 * n_tiles;
     const uint32_t* parts = static_cast<const uint32_t*>(scratch);
@@ -901,7 +896,7 @@ hipError_t launch_head_presplit(const void* W, int32_t wtype, const float* bias,
                                                           split_inv_offset(R, n_vocab))
                                : nullptr;
     return mfma_dispatch(W, wtype, bias, parts, inv, n_tiles, out0, nullptr, ld_out, n_rows,
-                         n_vocab, n_embd, stream, kz, gelu_out ? 1 : 0, out_parts, out_inv);
+                         n_vocab, n_embd, stream, kz, gelu_out ? 1 : 0, out_parts, out_inv, kv);
 }
 
 hipError_t launch_head_gemv_norm(const void* W, int32_t wtype, const float* bias,

@@ -146,15 +146,28 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
                          const float* hidden1, int64_t ld_hidden, float* out0, float* out1,
                          int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                          void* scratch, hipStream_t stream, int kz, bool gelu_out);
+// A q|k|v product of n_embd = n_head * 64 columns each whose k and v go
+// straight to their rows' cache slots and positions (rows with act[r] == 0
+// nowhere) instead of to the output rows; kc set where a product does so.
+struct KvOut {
+    float* kc;
+    float* vc;
+    const int32_t* positions;
+    const int32_t* slots;
+    const int32_t* act;
+    int32_t layer, n_layer, n_head, n_ctx;
+};
+
 // The matrix-core products of n_rows rows already split into `scratch` by
 // their producer (cbx_split.h's layout, n_rows padded to whole 16-row tiles):
 // launch_head_k without its split launch (one row set, any number of rows).
 // out_split set (no K split, n_vocab a multiple of 32): the outputs go there
-// split for the next product (rows of n_vocab) instead of to out0.
+// split for the next product (rows of n_vocab) instead of to out0.  kv.kc set
+// (no K split, no gelu): a q|k|v product.
 hipError_t launch_head_presplit(const void* W, int32_t wtype, const float* bias, float* out0,
                                 int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                                 const void* scratch, hipStream_t stream, int kz,
-                                bool gelu_out, void* out_split = nullptr);
+                                bool gelu_out, void* out_split, const KvOut& kv);
 
 // The same for many rows (cbx_tile.hip; head_uses_tiles: the rows and widths it
 // takes): the weights unpacked into `scratch` (device memory of
@@ -164,7 +177,7 @@ size_t tile_scratch_bytes(int32_t n_rows, int32_t n_vocab, int32_t n_embd);
 hipError_t launch_head_tiles(const void* W, int32_t wtype, const float* bias, float* out,
                              int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                              const void* split, void* scratch, hipStream_t stream, bool gelu_out,
-                             void* out_split);
+                             void* out_split, const KvOut& kv);
 
 // The T3 layer's residual add and layer norm folded into the mat-vec product
 // that consumes them (1 or 2 rows of n_embd, a multiple of 256, at most

@@ -85,7 +85,12 @@ struct TileArgs {
     int gelu_out;
     uint32_t* out_parts;   // when set, the outputs go there instead, split
     float* out_inv;
+    KvOut kv;              // a q|k|v product
 };
+
+// What a product's outputs become: fp32 rows, the next product's split rows,
+// or q rows beside k and v in the caches.
+enum class Out { kRows, kSplit, kQkv };
 
 typedef int32_t i4 __attribute__((ext_vector_type(4)));
 
@@ -127,7 +132,7 @@ __device__ __forceinline__ void wait_stage() {
 // DQ: quantized weights (their blocks' scales); F16 weights have none.
 constexpr int kFold = 8;
 
-template <bool DQ, int NT, int NC, int RW, int ST, bool SPLIT>
+template <bool DQ, int NT, int NC, int RW, int ST, Out OUT>
 __global__ __launch_bounds__(256 * RW, 2) void head_tile(TileArgs a) {
     constexpr int W = 4 * RW, WT = NT * RW, WC = 4 * NC;  // waves, row and output tiles
     static_assert(2 * WT % W == 0 && WC % W == 0 && NC % 2 == 0, "whole loads per wave, whole output blocks");
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(256 * RW, 2) void head_tile(TileArgs a) {
                 x[c][i] = __fadd_rn(tot[t][c][i], bias[c]);
                 if (a.gelu_out) x[c][i] = t3_gelu_f(x[c][i]);
             }
-        if constexpr (SPLIT) {  // n_vocab a multiple of 32: whole blocks in or out
+        if constexpr (OUT == Out::kSplit) {  // n_vocab a multiple of 32: whole blocks in or out
             const int nb_out = a.n_vocab / 32;
 #pragma unroll
             for (int c = 0; c < NC; c += 2) {
@@ -321,10 +326,16 @@ __global__ __launch_bounds__(256 * RW, 2) void head_tile(TileArgs a) {
                 const int rr = 16 * (T0 + T) + 4 * g + i;
                 if (rr >= a.n_rows) continue;
                 float* const o = a.out + (int64_t)rr * a.ld_out;
+                float* kvp = nullptr;
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
                     const int v = 16 * (C0 + c) + m;
-                    if (v < a.n_vocab) o[v] = x[c][i];
+                    if (OUT == Out::kQkv && 3 * 16 * (C0 + c) >= a.n_vocab) {
+                        if (c % 2 == 0) kvp = v < a.n_vocab ? kv_place(a.kv, rr, v) : nullptr;
+                        if (kvp) kvp[16 * (c % 2)] = x[c][i];
+                    } else if (v < a.n_vocab) {
+                        o[v] = x[c][i];
+                    }
                 }
             }
         }
@@ -345,9 +356,11 @@ hipError_t launch_tile(TileArgs a, hipStream_t st) {
     a.n_cg = (a.n_vocab + 64 * NC - 1) / (64 * NC);
     const dim3 grid((unsigned)((a.n_tiles + NT * RW - 1) / (NT * RW)) * (unsigned)a.n_cg);
     if (a.out_parts)
-        hipLaunchKernelGGL((head_tile<DQ, NT, NC, RW, ST, true>), grid, dim3(256 * RW), 0, st, a);
+        hipLaunchKernelGGL((head_tile<DQ, NT, NC, RW, ST, Out::kSplit>), grid, dim3(256 * RW), 0, st, a);
+    else if (a.kv.kc)
+        hipLaunchKernelGGL((head_tile<DQ, NT, NC, RW, ST, Out::kQkv>), grid, dim3(256 * RW), 0, st, a);
     else
-        hipLaunchKernelGGL((head_tile<DQ, NT, NC, RW, ST, false>), grid, dim3(256 * RW), 0, st, a);
+        hipLaunchKernelGGL((head_tile<DQ, NT, NC, RW, ST, Out::kRows>), grid, dim3(256 * RW), 0, st, a);
     return hipGetLastError();
 }
 
@@ -380,8 +393,9 @@ bool head_uses_tiles(int32_t n_rows, int32_t n_embd) {
 hipError_t launch_head_tiles(const void* W, int32_t wtype, const float* bias, float* out,
                              int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                              const void* split, void* scratch, hipStream_t st, bool gelu_out,
-                             void* out_split) {
-    if (!split || !scratch || !head_uses_tiles(n_rows, n_embd) || (out_split && n_vocab % 32 != 0))
+                             void* out_split, const KvOut& kv) {
+    if (!split || !scratch || !head_uses_tiles(n_rows, n_embd) || (out_split && n_vocab % 32 != 0) ||
+        (kv.kc && (out_split || gelu_out || n_vocab != 3 * 64 * kv.n_head)))
         return hipErrorInvalidValue;
     const int nball = n_embd / 32, n_tiles = (n_rows + 15) / 16;
     u4v* const wq = static_cast<u4v*>(scratch);
@@ -414,6 +428,7 @@ hipError_t launch_head_tiles(const void* W, int32_t wtype, const float* bias, fl
     a.out_inv = out_split ? reinterpret_cast<float*>(static_cast<char*>(out_split) +
                                                      split_inv_offset(16 * n_tiles, n_vocab))
                           : nullptr;
+    a.kv = kv;
     return wtype == CBX_WTYPE_F16 ? launch_tiles<false>(a, st) : launch_tiles<true>(a, st);
 }
 

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "cbx_internal.h"
 #include "cbx_split.h"
 #include "../../include/cbx_sampler.h"
 
@@ -115,6 +116,16 @@ __device__ __forceinline__ void store_split_tile(uint32_t* out_parts, float* out
         }
         if (in && m == 0) out_inv[split_inv_index(T, mrow, nb_out, blk)] = sinv;
     }
+}
+
+// Where k or v of row r, column v >= n of a q|k|v product of n columns each
+// goes (NULL: nowhere); every 32 columns from a multiple of 32 lie in one head.
+__device__ __forceinline__ float* kv_place(const KvOut& kv, int r, int v) {
+    if (!kv.act[r]) return nullptr;
+    const int n = kv.n_head * 64, c = v - n < n ? v - n : v - 2 * n;
+    return (v < 2 * n ? kv.kc : kv.vc) +
+           ((((int64_t)kv.slots[r] * kv.n_layer + kv.layer) * kv.n_head + (c >> 6)) * kv.n_ctx +
+            kv.positions[r]) * 64 + (c & 63);
 }
 
 }  // namespace cbx

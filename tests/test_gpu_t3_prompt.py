@@ -162,13 +162,15 @@ def test_nonfinite_row_stays_in_its_stream(small, lens, bad):
             assert np.array_equal(got[i], clean[i]), (b, p)
 
 
-# 1024 rows is where the products take large tiles; 8 x 1025 rows give c_attn
+# 672 rows is where head_mfma's c_attn takes two or four row tiles (q rows and
+# the caches its outputs), 1024 rows where the products take large tiles; 8 x 1025 rows give c_attn
 # and c_fc (768 and 1024 outputs) enough workgroups of 128 x 128, attn c_proj not
 @pytest.mark.parametrize("wtype,lens", [
     (O.WTYPE_Q4_0, (64,) * 16), (O.WTYPE_F16, (37,) * 30), (O.WTYPE_Q5_0, (1,) * 1023 + (18,)),
+    (O.WTYPE_Q8_0, (100,) * 8), (O.WTYPE_F16, (71,) * 10), (O.WTYPE_Q4_0, (75,) * 10),
     (O.WTYPE_Q8_0, (100,) * 82), (O.WTYPE_F16, (410,) * 20), (O.WTYPE_Q4_0, (391,) * 21)])
 def test_many_rows_products(small, wtype, lens):
-    """The tiled products, every format, whole and partial row tiles."""
+    """The products of many rows, every format, whole and partial row tiles."""
     torch, s = small[:2]
     dm, rm = model(torch, pkg.load(), wtype)
     rng = np.random.default_rng(len(lens))
