@@ -769,17 +769,20 @@ hipError_t launch_mfma(const void* W, const float* bias, const uint32_t* parts, 
 }
 
 // The matrix-core products on split activations: one row tile per workgroup
-// where two would leave fewer than 512 workgroups (narrow outputs, few rows:
-// the T3 layer products), the K is split or the outputs are split for the
-// next product; else two row tiles per workgroup for Q4_0 and for at most
-// two tiles.
+// where two would leave fewer than 512 workgroups (768 with split outputs, whose
+// end is longer; narrow outputs, few rows: the T3 layer products) or the K is split; else two row tiles per workgroup
+// for Q4_0 and for at most two tiles.  us per prompt pass with one tile / two
+// for c_fc too (split outputs, 4096 wide): 251 rows Q4_0 1720 / 1700, Q8_0 2109 /
+// 2045, F16 2525 / 2332, about 900 rows Q4_0 4244 / 4109, 128 rows (512
+// workgroups of two) 1216 / 1223; with two tiles beside a
+// K split 40 rows lose (943 / 985).
 hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const uint32_t* parts,
                          const float* inv, int n_tiles, float* out0, float* out1, int64_t ld_out,
                          int32_t n_rows, int32_t n_vocab, int32_t n_embd, hipStream_t stream,
                          int kz, int gelu_out, uint32_t* out_parts = nullptr,
                          float* out_inv = nullptr, const KvOut& kv = KvOut{}) {
-    const bool one = (int64_t)((n_vocab + 31) / 32) * ((n_tiles + 1) / 2) < 512 || kz > 1 ||
-                     gelu_out || out_parts;
+    const bool one = (int64_t)((n_vocab + 31) / 32) * ((n_tiles + 1) / 2) < (out_parts ? 768 : 512) ||
+                     kz > 1;
     const bool two = wtype == CBX_WTYPE_Q4_0 || wtype == CBX_WTYPE_Q5_0 || n_tiles <= 2;
     auto run = [&](auto wt) {
         constexpr int WT = decltype(wt)::value;

@@ -57,21 +57,22 @@ __device__ __forceinline__ void split_store(uint32_t* parts, int T, int m, int n
 // The T3 MLP's gelu, tanh form (Hendrycks and Gimpel; ggml_gelu's):
 // 0.5 x (1 + tanh(w)) with w = sqrt(2/pi) x (1 + 0.044715 x^2), taken as
 // x / (1 + exp(-2 w)), which is the same function without the cancellation
-// of 1 + tanh(w) at negative w.  exp through 2^t, t = -2 w log2(e), with the
-// rounding of t carried (an error of t is one of the whole result, |t| times
-// over); t is bounded where 2^t is 0 or infinite anyway, so that the
-// remainder stays finite.  About 20 instructions (tanhf: about 60), the
-// largest part of a c_fc tile's end.
+// of 1 + tanh(w) at negative w.  exp as 2^t, t = x (A x^2 + B) = -2 w log2(e),
+// with the rounding of the product carried; x is bounded in t where the
+// quotient is x or x 2^-122 anyway, so that 1 + e and its reciprocal stay
+// finite; the quotient by the approximate reciprocal takes one remainder
+// step.  About 20 instructions (tanhf: about 60), the largest part of a c_fc
+// tile's end.
 __device__ __forceinline__ float t3_gelu_f(float x) {
-    const float c = 0.7978845608028654f;  // sqrt(2 / pi)
-    const float kL = -2.8853900817779268f, kLlo = -2.8853900817779268 - (double)-2.8853900817779268f;
-    const float w =
-        __fmul_rn(__fmul_rn(c, x), __fadd_rn(1.0f, __fmul_rn(__fmul_rn(0.044715f, x), x)));
-    const float wc = fminf(fmaxf(w, -60.0f), 60.0f);  // t within +-174
-    const float t = __fmul_rn(wc, kL);
-    const float r = __fmaf_rn(wc, kLlo, __fmaf_rn(wc, kL, -t));
-    const float e = __fmul_rn(__builtin_amdgcn_exp2f(t), __fmaf_rn(r, 0.6931471805599453f, 1.0f));
-    return __fmul_rn(x, __builtin_amdgcn_rcpf(__fadd_rn(1.0f, e)));
+    const double kB = -2.0 * 0.79788456080286535588 * 1.44269504088896340736;  // -2 sqrt(2/pi) log2(e)
+    const float xc = fminf(fmaxf(x, -9.9f), 9.9f);
+    const float u = __fmaf_rn((float)(0.044715 * kB), __fmul_rn(xc, xc), (float)kB);
+    const float t = __fmul_rn(xc, u);
+    const float p = __builtin_amdgcn_exp2f(t);
+    const float r = __fmul_rn(__fmaf_rn(xc, u, -t), 0.6931471805599453f);
+    const float d = __fadd_rn(1.0f, __fmaf_rn(p, r, p));
+    const float y = __builtin_amdgcn_rcpf(d), q = __fmul_rn(x, y);
+    return __fmaf_rn(__fmaf_rn(-q, d, x), y, q);
 }
 
 // A DPP lane exchange within each 16-lane row (ctrl a compile-time DPP code).
