@@ -20,17 +20,7 @@ struct cbx_sampler {
     int32_t max_history = 0;
     size_t lds_limit = 0;
     hipStream_t stream = nullptr;
-    // device buffers for single-row calls
-    float* d_logits = nullptr;
-    float* d_uncond = nullptr;
-    int32_t* d_hist = nullptr;
-    int32_t* d_hist_len = nullptr;
-    cbx_params* d_params = nullptr;
-    uint32_t* d_allowed = nullptr;
-    uint8_t* d_force = nullptr;
-    double* d_u = nullptr;
-    int32_t* d_token = nullptr;
-    uint32_t* d_info = nullptr;
+    // the single-row calls' probabilities
     float* d_probs = nullptr;
     // redo lists (rows over a launch's survivor capacity): batched calls, and
     // the single-row calls on the handle's own stream
@@ -47,15 +37,23 @@ struct cbx_sampler {
     // the T3 decode step's workspace, grown on demand
     void* d_t3 = nullptr;
     size_t t3_bytes = 0;
-    // pinned host staging for the small per-call inputs/outputs
-    struct Small {
+    // Pinned host memory that the single-row kernels read and write in place
+    // (coherent: nothing of an earlier call stays in a cache): the row, the
+    // unconditional row, the history, the allowed words, then the rest.  Over
+    // the bus the kernel's own loads of a 26 KB row cost less than a copy
+    // each for up to eight inputs and two outputs (us per call at V = 6563, 256 ids:
+    // 62 -> 35; with CFG at V = 8194 75 -> 41; V = 32768 78 -> 51).
+    struct Row {
         cbx_params params;
         double u;
         int32_t hist_len;
         int32_t token;
         uint32_t info;
         uint8_t force;
-    }* h_small = nullptr;
+    };
+    char* h_row = nullptr;
+    char* d_row = nullptr;  // the same memory as the device addresses it
+    size_t row_uncond = 0, row_hist = 0, row_allowed = 0, row_rest = 0;
 };
 
 namespace {
@@ -117,22 +115,12 @@ struct DeviceGuard {
 void release(cbx_sampler* s) {
     DeviceGuard g(s->device);
     if (s->stream) (void)hipStreamSynchronize(s->stream);
-    (void)hipFree(s->d_logits);
-    (void)hipFree(s->d_uncond);
-    (void)hipFree(s->d_hist);
-    (void)hipFree(s->d_hist_len);
-    (void)hipFree(s->d_params);
-    (void)hipFree(s->d_allowed);
-    (void)hipFree(s->d_force);
-    (void)hipFree(s->d_u);
-    (void)hipFree(s->d_token);
-    (void)hipFree(s->d_info);
     (void)hipFree(s->d_probs);
     (void)hipFree(s->d_redo);
     (void)hipFree(s->d_redo_row);
     (void)hipFree(s->d_head);
     (void)hipFree(s->d_t3);
-    if (s->h_small) (void)hipHostFree(s->h_small);
+    if (s->h_row) (void)hipHostFree(s->h_row);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
 }
@@ -222,16 +210,6 @@ int cbx_sampler_create(cbx_sampler** out, int32_t device, int32_t max_vocab, int
     const size_t W = (size_t)(max_vocab + 31) / 32;
     const size_t h = (size_t)(max_history > 0 ? max_history : 1);
     e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc(&s->d_logits, sizeof(float) * max_vocab);
-    if (e == hipSuccess) e = hipMalloc(&s->d_uncond, sizeof(float) * max_vocab);
-    if (e == hipSuccess) e = hipMalloc(&s->d_hist, sizeof(int32_t) * h);
-    if (e == hipSuccess) e = hipMalloc(&s->d_hist_len, sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&s->d_params, sizeof(cbx_params));
-    if (e == hipSuccess) e = hipMalloc(&s->d_allowed, sizeof(uint32_t) * W);
-    if (e == hipSuccess) e = hipMalloc(&s->d_force, 1);
-    if (e == hipSuccess) e = hipMalloc(&s->d_u, sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&s->d_token, sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&s->d_info, sizeof(uint32_t));
     if (e == hipSuccess) e = hipMalloc(&s->d_probs, sizeof(float) * max_vocab);
     if (e == hipSuccess) e = hipMalloc(&s->d_redo, sizeof(int32_t) * cbx::kRedoWords);
     if (e == hipSuccess) e = hipMalloc(&s->d_redo_row, sizeof(int32_t) * 3);
@@ -243,7 +221,15 @@ int cbx_sampler_create(cbx_sampler** out, int32_t device, int32_t max_vocab, int
     // the lists start empty; each redo pass leaves them empty again
     if (e == hipSuccess) e = hipMemset(s->d_redo, 0, sizeof(int32_t) * cbx::kRedoWords);
     if (e == hipSuccess) e = hipMemset(s->d_redo_row, 0, sizeof(int32_t) * 3);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_small, sizeof(cbx_sampler::Small));
+    const auto whole = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    s->row_uncond = whole(sizeof(float) * max_vocab);
+    s->row_hist = 2 * s->row_uncond;
+    s->row_allowed = s->row_hist + whole(sizeof(int32_t) * h);
+    s->row_rest = s->row_allowed + whole(sizeof(uint32_t) * W);
+    if (e == hipSuccess)
+        e = hipHostMalloc((void**)&s->h_row, s->row_rest + sizeof(cbx_sampler::Row),
+                          hipHostMallocMapped | hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&s->d_row, s->h_row, 0);
     if (e == hipSuccess) e = static_scratch(device, &s->static_redo);
     if (e != hipSuccess) {
         release(s);
@@ -284,51 +270,43 @@ int cbx_sample_row_ex(cbx_sampler* s, const float* logits, const float* logits_u
     if (!(u >= 0.0 && u < 1.0)) return fail(CBX_ERR_INVALID, "cbx_sample_row: u outside [0, 1)");
     DeviceGuard g(s->device);
     hipStream_t st = s->stream;
-    cbx_sampler::Small* hs = s->h_small;
+    char* const hr = s->h_row;
+    cbx_sampler::Row* const hs = reinterpret_cast<cbx_sampler::Row*>(hr + s->row_rest);
     hs->params = *params;
     hs->u = u;
     hs->hist_len = n_history;
     hs->force = force_stop ? 1 : 0;
     const size_t W = (size_t)(n_vocab + 31) / 32;
-    CBX_HIP(hipMemcpyAsync(s->d_logits, logits, sizeof(float) * n_vocab, hipMemcpyHostToDevice, st));
-    if (logits_uncond)
-        CBX_HIP(hipMemcpyAsync(s->d_uncond, logits_uncond, sizeof(float) * n_vocab,
-                               hipMemcpyHostToDevice, st));
-    if (n_history > 0)
-        CBX_HIP(hipMemcpyAsync(s->d_hist, history, sizeof(int32_t) * n_history,
-                               hipMemcpyHostToDevice, st));
-    if (allowed)
-        CBX_HIP(hipMemcpyAsync(s->d_allowed, allowed, sizeof(uint32_t) * W, hipMemcpyHostToDevice, st));
-    CBX_HIP(hipMemcpyAsync(s->d_params, &hs->params, sizeof(cbx_params), hipMemcpyHostToDevice, st));
-    CBX_HIP(hipMemcpyAsync(s->d_u, &hs->u, sizeof(double), hipMemcpyHostToDevice, st));
-    CBX_HIP(hipMemcpyAsync(s->d_hist_len, &hs->hist_len, sizeof(int32_t), hipMemcpyHostToDevice, st));
-    CBX_HIP(hipMemcpyAsync(s->d_force, &hs->force, 1, hipMemcpyHostToDevice, st));
+    std::memcpy(hr, logits, sizeof(float) * n_vocab);
+    if (logits_uncond) std::memcpy(hr + s->row_uncond, logits_uncond, sizeof(float) * n_vocab);
+    if (n_history > 0) std::memcpy(hr + s->row_hist, history, sizeof(int32_t) * n_history);
+    if (allowed) std::memcpy(hr + s->row_allowed, allowed, sizeof(uint32_t) * W);
+    char* const dr = s->d_row;
+    cbx_sampler::Row* const ds = reinterpret_cast<cbx_sampler::Row*>(dr + s->row_rest);
 
     cbx::KernelArgs a{};
     a.n_rows = 1;
     a.n_vocab = n_vocab;
     a.n_steps = 1;
     a.stop_token = stop_token;
-    a.logits = s->d_logits;
+    a.logits = reinterpret_cast<const float*>(dr);
     a.ld_logits = n_vocab;
-    a.uncond = logits_uncond ? s->d_uncond : nullptr;
-    a.params = s->d_params;
-    a.history = s->d_hist;
-    a.history_len = s->d_hist_len;
+    a.uncond = logits_uncond ? reinterpret_cast<const float*>(dr + s->row_uncond) : nullptr;
+    a.params = &ds->params;
+    a.history = reinterpret_cast<const int32_t*>(dr + s->row_hist);
+    a.history_len = &ds->hist_len;
     a.ld_history = n_history;
-    a.allowed = allowed ? s->d_allowed : nullptr;
+    a.allowed = allowed ? reinterpret_cast<const uint32_t*>(dr + s->row_allowed) : nullptr;
     a.ld_allowed = (int64_t)W;
-    a.force_stop = s->d_force;
+    a.force_stop = &ds->force;
     a.draw_mode = CBX_DRAW_UNIFORM;
     a.cap = pick_cap(s, n_vocab, (params->top_k > 0 && params->top_k < n_vocab) ? params->top_k : 0);
-    a.uniforms = s->d_u;
-    a.tokens = s->d_token;
-    a.info = s->d_info;
+    a.uniforms = &ds->u;
+    a.tokens = &ds->token;
+    a.info = &ds->info;
     a.probs = probs_out ? s->d_probs : nullptr;
     a.ld_probs = n_vocab;
     CBX_HIP(launch_with_redo(pick_cap(s, n_vocab, 0), a, s->d_redo_row, s->latency_rows, st));
-    CBX_HIP(hipMemcpyAsync(&hs->token, s->d_token, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    CBX_HIP(hipMemcpyAsync(&hs->info, s->d_info, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     if (probs_out)
         CBX_HIP(hipMemcpyAsync(probs_out, s->d_probs, sizeof(float) * n_vocab, hipMemcpyDeviceToHost, st));
     CBX_HIP(hipStreamSynchronize(st));
