@@ -1,6 +1,6 @@
 """ctypes view of the test-only diagnostics library (tests/native/cbx_debug.h,
 built by `make -C tests/native`): the sampler's device exponential, Philox
-uniforms and exact running sums and the T3 MLP's gelu on caller-given inputs."""
+uniforms and exact running sums on caller-given inputs."""
 import ctypes
 import os
 
@@ -24,7 +24,6 @@ def lib():
         L.cbx_debug_philox.argtypes = [i32, u64, vp, u64, i32, vp, vp]
         L.cbx_debug_runsum.argtypes = [i32, vp, vp, vp, vp, i32, vp, vp, vp]
         L.cbx_debug_chainsum.argtypes = [i32, vp, vp, vp, i32, vp, vp, vp]
-        L.cbx_debug_gelu.argtypes = [i32, vp, vp, i64, vp]
         _lib = L
     return _lib
 
@@ -41,10 +40,6 @@ def _ok(rc, name):
 
 def expf(x, out, device=0):
     _ok(lib().cbx_debug_expf(device, x.data_ptr(), out.data_ptr(), x.numel(), _stream()), "expf")
-
-
-def gelu(x, out, device=0):
-    _ok(lib().cbx_debug_gelu(device, x.data_ptr(), out.data_ptr(), x.numel(), _stream()), "gelu")
 
 
 def runsum(terms, offsets, thr, desc, sums, hits, device=0):

@@ -1,4 +1,4 @@
-/* cbx_debug.h -- test-only diagnostics of the library's device building
+/* cbx_debug.h -- test-only diagnostics of the sampler's device building
  * blocks (tests/native/_build/libcbx_debug.so, built from
  * tests/native/cbx_debug.hip; not part of libcbx_sampler.so or its API).
  * Device memory, asynchronous on `stream`; `device` is made current for the
@@ -32,8 +32,6 @@ int cbx_debug_runsum(int32_t device, const float* terms, const int32_t* offsets,
  * terms per case; the case's sum starts from 0. */
 int cbx_debug_chainsum(int32_t device, const float* terms, const int32_t* offsets,
                        const float* thr, int32_t n_cases, float* sum, int32_t* hit, void* stream);
-/* The T3 MLP's gelu (t3_gelu_f, cbx_split.h), elementwise. */
-int cbx_debug_gelu(int32_t device, const float* in, float* out, int64_t n, void* stream);
 
 #ifdef __cplusplus
 }

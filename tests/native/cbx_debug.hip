@@ -1,11 +1,10 @@
 // cbx_debug.hip -- test-only diagnostics (libcbx_debug.so): the device
 // exponential, the device Philox uniforms and the two exact running-sum
-// evaluations of the sampler and the T3 MLP's gelu, run on caller-given inputs so the tests can
+// evaluations of the sampler, run on caller-given inputs so the tests can
 // compare them with the host (tests/native/cbx_debug.h).
 #include <hip/hip_runtime.h>
 
 #include "../../chatterbox.cpp_amd/csrc/cbx_sampler_wave.h"
-#include "../../chatterbox.cpp_amd/csrc/cbx_split.h"
 #include "cbx_debug.h"
 
 namespace cbx {
@@ -17,11 +16,6 @@ __global__ void debug_expf_kernel(const float* in, float* out, int64_t n) {
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) out[i] = expf_libm_branchless(in[i], tab);
-}
-
-__global__ void debug_gelu_kernel(const float* in, float* out, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = t3_gelu_f(in[i]);
 }
 
 __global__ void debug_philox_kernel(uint64_t seed, const uint64_t* sid, uint64_t step, int32_t n,
@@ -123,15 +117,6 @@ int cbx_debug_expf(int32_t device, const float* in, float* out, int64_t n, void*
     DevGuard g(device);
     const int64_t blocks = (n + 255) / 256;
     hipLaunchKernelGGL(cbx::debug_expf_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       (hipStream_t)stream, in, out, n);
-    return launch_done(device, hipGetLastError());
-}
-
-int cbx_debug_gelu(int32_t device, const float* in, float* out, int64_t n, void* stream) {
-    if (!in || !out || n < 0) return CBX_ERR_INVALID;
-    if (n == 0) return CBX_OK;
-    DevGuard g(device);
-    hipLaunchKernelGGL(cbx::debug_gelu_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, in, out, n);
     return launch_done(device, hipGetLastError());
 }

@@ -12,7 +12,7 @@ quotient, 2^-23; e below the smallest normal number counts as 0.
 import numpy as np
 import pytest
 
-import debug_lib as D
+import debug_t3_lib as D
 
 pytestmark = pytest.mark.gpu
 
