@@ -213,11 +213,6 @@ int cbx_sampler_create(cbx_sampler** out, int32_t device, int32_t max_vocab, int
     if (e == hipSuccess) e = hipMalloc(&s->d_probs, sizeof(float) * max_vocab);
     if (e == hipSuccess) e = hipMalloc(&s->d_redo, sizeof(int32_t) * cbx::kRedoWords);
     if (e == hipSuccess) e = hipMalloc(&s->d_redo_row, sizeof(int32_t) * 3);
-    // the head's split buffer, enough for every call of fewer than 16 rows
-    // that the mat-vec's LDS could hold (32 padded rows with CFG): such calls
-    // do not allocate
-    s->head_bytes = cbx::head_scratch_bytes(16, true, 2240);
-    if (e == hipSuccess) e = hipMalloc(&s->d_head, s->head_bytes);
     // the lists start empty; each redo pass leaves them empty again
     if (e == hipSuccess) e = hipMemset(s->d_redo, 0, sizeof(int32_t) * cbx::kRedoWords);
     if (e == hipSuccess) e = hipMemset(s->d_redo_row, 0, sizeof(int32_t) * 3);
@@ -490,8 +485,9 @@ int check_head(const char* fn, const cbx_head* h, int32_t n_rows, int32_t n_voca
 }
 
 // The handle's split buffer holds one call's activations at a time: head calls
-// on one handle are ordered on one stream (a larger call than any before
-// waits for the device while the buffer is replaced).
+// of 16 projected rows and more on one handle are ordered on one stream (a
+// larger call than any before waits for the device while the buffer is
+// replaced); smaller ones do not use it.
 int run_head(cbx_sampler* s, const cbx_head* h, int32_t n_rows, int32_t n_vocab,
              int64_t ld_logits, hipStream_t st) {
     const size_t need = cbx::head_scratch_bytes(n_rows, h->hidden_uncond != nullptr, h->n_embd);

@@ -8,12 +8,13 @@
 // little-endian word qh whose bit j is the fifth bit of element j, and the
 // nibbles as Q4_0's, w = (q - 16) d; Q8_0 blocks are d and 32 int8, w = q d).
 //
-// 7 rows and more run on the fp16 matrix cores in two launches:
-//  * head_split: each activation row r is scaled by a power of two 2^s_r (its
-//    largest magnitude to [2^14, 2^15)) and written as two fp16 parts,
-//    x 2^s = hi + lo + e with |e| <= 2^-23 |x 2^s| + 2^-25 (hi and lo rounded
-//    to nearest; the 2^-25 is lo's subnormal step, 2^-39 of the row's largest
-//    value), together with 2^-s_r, in the matrix-core operand order: for
+// 7 projected rows and more run on the fp16 matrix cores, from 16 in two
+// launches (fewer split their rows inside the second):
+//  * head_split: each block of 32 activations of a row is scaled by a power of
+//    two 2^s (its largest magnitude to [2^14, 2^15)) and written as two fp16
+//    parts, x 2^s = hi + lo + e with |e| <= 2^-23 |x 2^s| + 2^-25 (hi and lo
+//    rounded to nearest; the 2^-25 is lo's subnormal step, 2^-39 of the block's
+//    largest value), together with 2^-s, in the matrix-core operand order: for
 //    each 16-row tile and 32-weight block, the 64 lanes' 16 bytes of hi parts,
 //    then their 16 bytes of lo parts, so each operand load reads 1 KB
 //    contiguous (loads of 64-byte pieces of 16 rows were the kernel's limit).
@@ -23,9 +24,10 @@
 //    integers (n - 8, q - 16 or q, exact in fp16) with each block's product scaled by its d
 //    in fp32.  Products of fp16 values are exact in fp32; sums are the
 //    matrix core's fp32.  Wave w takes the w-th of KS runs of 32-weight
-//    blocks along n_embd, and the KS partial tiles are added in wave order
-//    through LDS (a fixed order: results do not depend on scheduling); the
-//    sum is scaled back by 2^-s_r (exact) and the bias added.
+//    blocks along n_embd, each block's products scaled back by their rows'
+//    2^-s (exact) as they are added, and the KS partial tiles are added in
+//    wave order through LDS (a fixed order: results do not depend on
+//    scheduling), then the bias.
 // Lane l feeds A[l%16][8(l/16) ..] and B[8(l/16) ..][l%16] (the same k on
 // both operands, so a tile's products are sums over every k) and holds
 // D[4(l/16)+i][l%16]: hidden row 4(l/16)+i of the tile, vocab id l%16.
@@ -143,13 +145,27 @@ constexpr int RING = 2;
 // (rows of n_vocab values: this workgroup's 32 outputs are block blockIdx.x
 // of each of its rows) instead of fp32 rows.
 // KV: a q|k|v product, its k and v stored in the caches (kv_place).
-template <int WT, int NT, bool KV>
+// SELF (at most 15 rows: one tile per row set): the rows themselves (`rows`)
+// instead of their split; a block's values are split as the block is taken, by
+// the operations of head_split and with the same results.  The split (about 70
+// VALU instructions per block) is repeated by every workgroup, but no launch
+// comes before the product and no memory is shared between calls: us per call
+// of 7 rows at V = 6563, n_embd = 1024, with a split launch / here, Q4_0 10.9 / 7.0,
+// Q8_0 10.9 / 7.6, F16 10.9 / 7.5; V = 32768 (1024 workgroups), 12 rows, Q4_0 14.3 /
+// 18.0, F16 25.3 / 24.8.
+struct HeadRows {
+    const float* set0;
+    const float* set1;
+    int64_t ld;
+};
+template <int WT, int NT, bool KV, bool SELF>
 __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == CBX_WTYPE_Q4_0 ? 4 : 1))) void head_mfma(const void* W, const float* bias,
                                                      const uint32_t* parts, const float* inv,
                                                      int n_tiles, float* out0, float* out1,
                                                      int64_t ld_out, int n_rows, int n_vocab,
                                                      int n_embd, int64_t zstride, int gelu_out,
-                                                     uint32_t* out_parts, float* out_inv, KvOut kv) {
+                                                     uint32_t* out_parts, float* out_inv, KvOut kv,
+                                                     HeadRows rows) {
     constexpr int BB = block_bytes<WT>();
     // Weights are staged per wave in chunks of CB blocks: for each of the 32
     // vocab rows the chunk's CB * BB bytes are contiguous, so whole-row dword
@@ -169,8 +185,14 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == C
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<void*>(W), (short)0, (int)wbytes, kBufWord3);
     const int pbytes = n_tiles * 16 * n_embd * 4;
+    // SELF: a set's rows, to the end of the last
+    const int rbytes = (int)(((int64_t)(n_rows - 1) * rows.ld + n_embd) * 4);
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint32_t*>(parts), (short)0, pbytes, kBufWord3);
+        SELF ? const_cast<float*>(NT == 1 && blockIdx.y ? rows.set1 : rows.set0)
+             : reinterpret_cast<float*>(const_cast<uint32_t*>(parts)),
+        (short)0, SELF ? rbytes : pbytes, kBufWord3);
+    const __amdgpu_buffer_rsrc_t rp1 = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(rows.set1), (short)0, SELF && rows.set1 ? rbytes : 0, kBufWord3);
     const int sbytes = n_tiles * 16 * (n_embd / 32) * 4;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(inv), (short)0, sbytes, kBufWord3);
@@ -185,6 +207,10 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == C
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int T = blockIdx.y * NT + t;
+        if constexpr (SELF) {  // row m's group g; rows past the set's last read zeros
+            hoff[t] = m < n_rows ? (uint32_t)(m * rows.ld + 8 * g) * 4u : 0x80000000u;
+            continue;
+        }
         hoff[t] = T < n_tiles ? (uint32_t)(T * nball * 512 + 4 * lane) * 4u : (uint32_t)pbytes;
         // the scales of rows 4g .. 4g + 3 (the rows of this lane's outputs)
         soff[t] = T < n_tiles ? (uint32_t)split_inv_index(T, 4 * g, nball, 0) * 4u : (uint32_t)sbytes;
@@ -208,6 +234,13 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == C
     auto load = [&](int kb, int r) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
+            if constexpr (SELF) {
+                const uint32_t o = hoff[t] + (uint32_t)kb * 128u;
+                const __amdgpu_buffer_rsrc_t rr = t == 0 ? rp : rp1;
+                ph[r][t] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(rr, o, 0, 0));
+                pl[r][t] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(rr, o + 16, 0, 0));
+                continue;
+            }
             const uint32_t o = hoff[t] + (uint32_t)kb * 2048u;
             ph[r][t] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, 0));
             pl[r][t] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(rp, o + 1024, 0, 0));
@@ -217,9 +250,31 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(WT == C
 #pragma unroll
     for (int r = 0; r + 1 < RING; ++r) load(kb0 + r, r);
     uint32_t* const sw = stage[wave];
+    // SELF: set r's values split in place, the block's scale from the four
+    // lanes of a row, then sv as the lanes of a product tile hold it
+    auto split = [&](int r) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            float x[8], mx = 0.0f, scl, sinv;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x[e] = __builtin_bit_cast(f4, ph[r][t])[e];
+                x[4 + e] = __builtin_bit_cast(f4, pl[r][t])[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[e]));
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            split_scale(mx, scl, sinv);
+            split_group(x, scl, ph[r][t], pl[r][t]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sv[r][t][i] = __shfl(sinv, 4 * g + i);
+        }
+    };
     // one block: its weights from the staged chunk, the next block's parts
     // requested, then the products
     auto block = [&](int kb, int kbc, int sha, int shb, int r) {
+        if constexpr (SELF) split(r);
         const u4v* const ch = ph[r];
         const u4v* const cl = pl[r];
         const f4* const sc = sv[r];
@@ -765,20 +820,20 @@ hipError_t launch_gemv_r(const void* W, const float* bias, const float* hidden0,
 template <int WT, int NT>
 hipError_t launch_mfma(const void* W, const float* bias, const uint32_t* parts, const float* inv,
                        int n_tiles, float* out0, float* out1, int64_t ld_out, int n_rows,
-                       int n_vocab, int n_embd, hipStream_t stream, int kz = 1,
-                       int gelu_out = 0, uint32_t* out_parts = nullptr,
-                       float* out_inv = nullptr, const KvOut& kv = KvOut{}) {
+                       int n_vocab, int n_embd, hipStream_t stream, int kz, int gelu_out,
+                       uint32_t* out_parts, float* out_inv, const KvOut& kv,
+                       const HeadRows& rows) {
     const dim3 grid((unsigned)((n_vocab + 31) / 32), (unsigned)((n_tiles + NT - 1) / NT),
                     (unsigned)kz);
-    if (kv.kc)
-        hipLaunchKernelGGL((head_mfma<WT, NT, true>), grid, dim3(64 * KS), 0, stream, W, bias,
-                           parts, inv, n_tiles, out0, out1, ld_out, n_rows, n_vocab, n_embd,
-                           (int64_t)n_rows * ld_out, 0, nullptr, nullptr, kv);
-    else
-        hipLaunchKernelGGL((head_mfma<WT, NT, false>), grid, dim3(64 * KS), 0, stream, W, bias,
-                           parts, inv, n_tiles, out0, out1, ld_out, n_rows, n_vocab, n_embd,
-                           (int64_t)n_rows * ld_out, gelu_out, out_parts, out_inv, kv);
-    return hipGetLastError();
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * KS), 0, stream, W, bias, parts, inv, n_tiles,
+                           out0, out1, ld_out, n_rows, n_vocab, n_embd, (int64_t)n_rows * ld_out,
+                           gelu_out, out_parts, out_inv, kv, rows);
+        return hipGetLastError();
+    };
+    if constexpr (NT <= 2)
+        if (rows.set0) return go(head_mfma<WT, NT, false, true>);
+    return kv.kc ? go(head_mfma<WT, NT, true, false>) : go(head_mfma<WT, NT, false, false>);
 }
 
 // The matrix-core products on split activations: one row tile per workgroup
@@ -793,7 +848,8 @@ hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const 
                          const float* inv, int n_tiles, float* out0, float* out1, int64_t ld_out,
                          int32_t n_rows, int32_t n_vocab, int32_t n_embd, hipStream_t stream,
                          int kz, int gelu_out, uint32_t* out_parts = nullptr,
-                         float* out_inv = nullptr, const KvOut& kv = KvOut{}) {
+                         float* out_inv = nullptr, const KvOut& kv = KvOut{},
+                         const HeadRows& rows = HeadRows{}) {
     const bool one = (int64_t)((n_vocab + 31) / 32) * ((n_tiles + 1) / 2) < (out_parts ? 768 : 512) ||
                      kz > 1;
     const bool two = wtype == CBX_WTYPE_Q4_0 || wtype == CBX_WTYPE_Q5_0 || n_tiles <= 2;
@@ -802,7 +858,7 @@ hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const 
         auto go = [&](auto nt) {
             return launch_mfma<WT, decltype(nt)::value>(W, bias, parts, inv, n_tiles, out0, out1,
                                                         ld_out, n_rows, n_vocab, n_embd, stream,
-                                                        kz, gelu_out, out_parts, out_inv, kv);
+                                                        kz, gelu_out, out_parts, out_inv, kv, rows);
         };
         if (one) return go(std::integral_constant<int, 1>{});
         if constexpr (WT == CBX_WTYPE_F16 || WT == CBX_WTYPE_Q8_0)
@@ -820,18 +876,23 @@ hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const 
 
 }  // namespace
 
-// The mat-vec's work grows with its rows, the matrix cores' does not below 16,
-// and their two launches take 11 us: us per call at V = 6563, n_embd = 1024,
-// mat-vec / matrix cores, 3 rows 7.6 / 11.1, 5 10.4 / 11.2, 7 12.2 / 11.2, 12
-// 19.2 / 11.2 (Q8_0; the other formats within 0.2).
+// The mat-vec's work grows with its rows, the matrix cores' does not below 16:
+// us per call at V = 6563, n_embd = 1024, mat-vec / matrix cores, 3 rows 7.4 /
+// 7.6, 6 11.3 / 7.6, 7 12.2 / 7.6, 15 23.0 / 7.6 (Q8_0; Q4_0 7.0 on the matrix
+// cores, the others within 0.2).  Up to 6 rows the activations stay fp32
+// operands (a guided batch of 3 and fewer), so their results are the mat-vec's.
 bool head_uses_gemv(int32_t n_rows, bool cfg, int32_t n_embd) {
     const int R = cfg ? 2 * n_rows : n_rows;
     return R < 7 && (size_t)R * gemv_row_words(n_embd) * 4 <= 65536;
 }
 
+// Calls of fewer projected rows hold nothing in memory between launches, so
+// they may run on several streams of one handle at once.
+constexpr int kSelfRows = 16;
+
 size_t head_scratch_bytes(int32_t n_rows, bool cfg, int32_t n_embd) {
     const int n_tiles = ((n_rows + 15) / 16) * (cfg ? 2 : 1);
-    return head_uses_gemv(n_rows, cfg, n_embd) ? 0 : split_bytes(16 * n_tiles, n_embd);
+    return n_rows * (cfg ? 2 : 1) < kSelfRows ? 0 : split_bytes(16 * n_tiles, n_embd);
 }
 
 hipError_t launch_head(const void* W, int32_t wtype, const float* bias, const float* hidden0,
@@ -855,7 +916,8 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
                          int64_t ld_out, int32_t n_rows, int32_t n_vocab, int32_t n_embd,
                          void* scratch, hipStream_t stream, int kz, bool gelu_out) {
     // fewer than 7 projected rows: the mat-vec (activations staged in LDS,
-    // at most 64 KiB of them), else the split and the 16-row matrix-core tiles
+    // at most 64 KiB of them), else the 16-row matrix-core tiles, from 16
+    // projected rows after a launch that splits them
     const bool cfg = hidden1 != nullptr;
     if (kz < 1 || (kz > 1 && (cfg || gelu_out || head_uses_gemv(n_rows, cfg, n_embd))))
         return hipErrorInvalidValue;  // a K split: one row set on the matrix cores, no gelu
@@ -881,8 +943,12 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
                 return hipErrorInvalidValue;
         }
     }
-    if (!scratch) return hipErrorInvalidValue;
     const int n_tiles = ((n_rows + 15) / 16) * (cfg ? 2 : 1), R = 16 * n_tiles;
+    if (n_rows * (cfg ? 2 : 1) < kSelfRows)
+        return mfma_dispatch(W, wtype, bias, nullptr, nullptr, n_tiles, out0, out1, ld_out, n_rows,
+                             n_vocab, n_embd, stream, kz, gelu_out ? 1 : 0, nullptr, nullptr,
+                             KvOut{}, HeadRows{hidden0, hidden1, ld_hidden});
+    if (!scratch) return hipErrorInvalidValue;
     uint32_t* parts = static_cast<uint32_t*>(scratch);
     float* inv = reinterpret_cast<float*>(static_cast<char*>(scratch) + split_inv_offset(R, n_embd));
     const int64_t groups = (int64_t)R * (n_embd / 8);

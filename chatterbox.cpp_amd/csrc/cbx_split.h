@@ -36,10 +36,9 @@ __device__ __forceinline__ void split_scale(float mx, float& sc, float& inv) {
     inv = __builtin_bit_cast(float, (uint32_t)(127 - s) << 23);
 }
 
-// Group j of row (T, m) from its 8 values x, scaled by sc, stored in place.
-__device__ __forceinline__ void split_store(uint32_t* parts, int T, int m, int nball, int j,
-                                            const float (&x)[8], float sc) {
-    split_u4 hi, lo;
+// A group's 8 values x, scaled by sc, as the operand's hi and lo parts.
+__device__ __forceinline__ void split_group(const float (&x)[8], float sc, split_u4& hi,
+                                            split_u4& lo) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const float y0 = __fmul_rn(x[2 * i], sc), y1 = __fmul_rn(x[2 * i + 1], sc);
@@ -49,6 +48,13 @@ __device__ __forceinline__ void split_store(uint32_t* parts, int T, int m, int n
         hi[i] = __builtin_bit_cast(uint32_t, split_h2{h0, h1});
         lo[i] = __builtin_bit_cast(uint32_t, split_h2{l0, l1});
     }
+}
+
+// Group j of row (T, m) from its 8 values x, scaled by sc, stored in place.
+__device__ __forceinline__ void split_store(uint32_t* parts, int T, int m, int nball, int j,
+                                            const float (&x)[8], float sc) {
+    split_u4 hi, lo;
+    split_group(x, sc, hi, lo);
     uint32_t* const o = parts + (int64_t)T * nball * 512 + 4 * m + (j >> 2) * 512 + 64 * (j & 3);
     *reinterpret_cast<split_u4*>(o) = hi;
     *reinterpret_cast<split_u4*>(o + 256) = lo;

@@ -207,12 +207,14 @@ typedef struct cbx_head {
 
 /* The projection alone for n_rows rows of hidden (and hidden_uncond) into
  * logits (and logits_uncond), row stride ld_logits >= n_vocab; weights as
- * the format defines them, exact products, fp32 sums.  From 16 projected rows
- * on, the fp16 matrix cores take each activation row scaled by a power of
- * two as two fp16 parts (each activation to 2^-23 relative plus 2^-39 of
- * its row's largest magnitude), held in a device buffer of the
- * handle that a call larger than any before it replaces (waiting for the
- * device): head calls on one handle are ordered on one stream.
+ * the format defines them, exact products, fp32 sums.  From 7 projected rows
+ * on (cond and uncond rows together; fewer where n_embd is too long for the
+ * mat-vec's LDS), the fp16 matrix cores take each activation, scaled by a power
+ * of two per 32 of its row, as two fp16 parts (to 2^-23 relative plus 2^-39 of
+ * the largest magnitude among the 32).  From 16 projected rows on, these are
+ * held in a device buffer of the handle that a call larger than any before it
+ * replaces (waiting for the device): such calls on one handle are ordered on
+ * one stream.  Smaller calls hold nothing in the handle.
  * Replaces the speech_head mul_mat of the T3 step (main.cpp:577).  Async. */
 int cbx_head_logits(cbx_sampler* s, const cbx_head* h, int32_t n_rows, int32_t n_vocab,
                     int64_t ld_logits, void* stream);
