@@ -544,7 +544,7 @@ __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
 // A masked key's weight is 0, and 0 times a V that is not finite would reach
 // rows that do not see that key: tiles that some row does not see whole look
 // for such values and, where one is found, add row by row with the unseen
-// keys' V at 0.
+// keys' V at 0, each row in the same order of adds.
 // KS = 4: the workgroup's four waves take the same rows and every fourth
 // pair of tiles, merged through LDS by the same rescaling in wave order
 // (small calls); KS = 1: each wave its own rows.
@@ -678,7 +678,7 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
                     const int li = __builtin_amdgcn_readlane(lim, i);
 #pragma unroll
                     for (int dt = 0; dt < 4; ++dt) {
-                        f4 add = f4{0.0f, 0.0f, 0.0f, 0.0f};
+                        f4 add = o[dt];
 #pragma unroll
                         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -688,7 +688,7 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
                             }
 #pragma unroll
                         for (int v = 0; v < 4; ++v)
-                            if (4 * g + v == i) o[dt][v] = __fadd_rn(o[dt][v], add[v]);
+                            if (4 * g + v == i) o[dt][v] = add[v];
                     }
                 }
             }

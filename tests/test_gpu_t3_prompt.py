@@ -162,6 +162,30 @@ def test_nonfinite_row_stays_in_its_stream(small, lens, bad):
             assert np.array_equal(got[i], clean[i]), (b, p)
 
 
+@pytest.mark.parametrize("lens,hit", [((180, 21), (0, 140)), ((70,) * 60, (1, 50))],
+                         ids=["split-keys", "group-per-wave"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_nonfinite_row_late_in_its_stream(small, lens, hit, bad):
+    """The same with rows in their streams' order, so that earlier rows of the
+    hit stream share its 16-row group, and the hit position past the first
+    pair of key tiles that its wave takes (sums already there to add to)."""
+    torch, s, dm, _ = small
+    rng = np.random.default_rng(12)
+    rows = arranged(lens, "streams", rng)
+    at = rows.index(hit)
+    assert at // 16 == (at - 2) // 16 and hit[1] >= (128 if len(rows) < 4096 else 32)
+    x = (rng.standard_normal((len(rows), N)) * 0.7).astype(np.float32)
+    print(f"[gpu-case] late nonfinite {bad} rows={len(rows)}", flush=True)
+    clean, _, _ = run(torch, s, dm, rows, x, len(lens), 200)
+    x[at, 3] = bad
+    got, _, _ = run(torch, s, dm, rows, x, len(lens), 200)
+    for i, (b, p) in enumerate(rows):
+        if b == hit[0] and p >= hit[1]:
+            assert np.isnan(got[i]).any()
+        else:
+            assert np.array_equal(got[i], clean[i]), (b, p)
+
+
 # 672 rows is where head_mfma's c_attn takes two or four row tiles (q rows and
 # the caches its outputs), 1024 rows where the products take large tiles; 8 x 1025 rows give c_attn
 # and c_fc (768 and 1024 outputs) enough workgroups of 128 x 128, attn c_proj not
