@@ -34,6 +34,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "cbx_group.h"
 #include "cbx_internal.h"
 #include "cbx_split.h"
 #include "cbx_weights.h"
@@ -61,7 +62,8 @@ struct NormArgs {
     const int32_t* tokens;
     int32_t* positions;
     const int32_t* state;
-    const int32_t* slots;  // prefill: the cache slot of each row (NULL: the row)
+    const int32_t* slots;  // prefill: the cache slot of each row
+    const int32_t* rows;   // prefill: the rows in groups of 16 (t3_group_rows; NULL: in order)
     int32_t n_slots;
     int32_t n_vocab, n_pos, n_ctx;
     int32_t* act;          // per row: 1 when the stream takes this step
@@ -290,7 +292,8 @@ struct AttnArgs {
     int32_t n_layer, layer, n_head, n_ctx;
     const int32_t* positions;
     const int32_t* act;
-    const int32_t* slots;  // prefill: the cache slot of each row (NULL: the row)
+    const int32_t* slots;  // prefill: the cache slot of each row
+    const int32_t* rows;   // prefill: the rows in groups of 16 (t3_group_rows; NULL: in order)
     float* out;            // [n_rows][n_embd]
     uint32_t* parts;       // when set, the rows go there instead, split for the
     float* inv;            //   next product (cbx_split.h), the scales here
@@ -540,7 +543,8 @@ __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
 // Each row has its running max, sum and outputs (rescaled as its max grows;
 // a tile in which a row sees no key leaves that row's as they are), so a
 // row's result does not depend on the rows beside it.  The 16 rows may belong
-// to any slots: one pass per distinct slot, the other rows' keys masked.
+// to any slots: one pass per distinct slot, the other rows' keys masked; the
+// caller's rows are grouped by slot first (t3_group_rows).
 // A masked key's weight is 0, and 0 times a V that is not finite would reach
 // rows that do not see that key: tiles that some row does not see whole look
 // for such values and, where one is found, add row by row with the unseen
@@ -553,16 +557,28 @@ __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
 // about 80); one prompt of 251 rows 24.5 -> 11 us.  32 rows per wave (half the
 // loads of K and V) measured 235: registers for two waves per SIMD, not three.
 template <int KS>
-__global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_rows) {
+__global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_rows,
+                                                            int n_groups) {
     constexpr int kWaves = 4, KT = 2;  // KT tiles of 16 keys per iteration
     static_assert(KS == 1 || KS == kWaves, "every wave its own rows, or all the same");
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int g = lane >> 4, c = lane & 15, h = blockIdx.y;
+    const int g = lane >> 4, c = lane & 15;
+    // grouped rows: a group's heads first, so that the empty groups come last
+    const int h = a.rows ? blockIdx.x : blockIdx.y;
+    const int wg = a.rows ? blockIdx.y : blockIdx.x;
     const int n = a.n_head * kHeadDim;
-    const int r0 = (KS == 1 ? (int)blockIdx.x * kWaves + w : (int)blockIdx.x) * 16;
-    if (r0 >= n_rows) return;  // whole waves, and only where no barrier follows (KS = 1)
-    const int rc = min(r0 + c, n_rows - 1);
-    const bool real = r0 + c < n_rows && a.act[rc] != 0;
+    const int group = KS == 1 ? wg * kWaves + w : wg;
+    // this lane's row (n_rows: none)
+    int row = 16 * group + c;
+    if (a.rows) {
+        const int at = group < n_groups ? a.rows[row] : -1;
+        row = at < 0 ? n_rows : at;
+    }
+    // an empty group: whole workgroups, or whole waves where no barrier
+    // follows (KS = 1)
+    if (!__ballot(row < n_rows)) return;
+    const int rc = min(row, n_rows - 1);
+    const bool real = row < n_rows && a.act[rc] != 0;
     const int pos = a.positions[rc], slot = a.slots[rc];
     f4 q[4], o[4];
     {
@@ -704,7 +720,7 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
             f4 x;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) x[dt] = on ? __fdiv_rn(o[dt][v], sv) : 0.0f;
-            attn_store4(a, n_rows, r0 + 4 * g + v, h, c, x);
+            attn_store4(a, n_rows, __shfl(row, 4 * g + v), h, c, x);
         }
     } else {
         // wave w joins the four waves' rows 4 g + w
@@ -734,7 +750,7 @@ __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_r
         const bool on = __shfl((int)real, i) != 0;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) at[dt] = on ? __fdiv_rn(at[dt], st) : 0.0f;
-        attn_store4(a, n_rows, r0 + i, h, c, at);
+        attn_store4(a, n_rows, __shfl(row, i), h, c, at);
     }
 }
 
@@ -749,14 +765,13 @@ hipError_t launch_norm_ept(const NormArgs& a, int n_rows, hipStream_t st) {
 // KS = 1: 1 x 251 rows 1.91 / 2.23, 1 x 700 3.77 / 4.29, 4 x 251 (1008 groups)
 // 4.49 / 4.53, 64 x 24 (1536) 6.10 / 5.90, 16 x 251 14.48 / 14.43, 48 x 290
 // 50.6 / 50.0.
-hipError_t launch_attn_tile(const AttnArgs& a, int n_rows, hipStream_t st) {
-    const int groups = (n_rows + 15) / 16;
-    if ((int64_t)groups * a.n_head < 1024)
-        hipLaunchKernelGGL(t3_attn_tile<4>, dim3((unsigned)groups, (unsigned)a.n_head),
-                           dim3(4 * kHeadDim), 0, st, a, n_rows);
-    else
-        hipLaunchKernelGGL(t3_attn_tile<1>, dim3((unsigned)((groups + 3) / 4), (unsigned)a.n_head),
-                           dim3(4 * kHeadDim), 0, st, a, n_rows);
+// n_groups: those of a.rows, or all rows in order.
+hipError_t launch_attn_tile(const AttnArgs& a, int n_rows, int n_groups, hipStream_t st) {
+    const bool split = (int64_t)((n_rows + 15) / 16) * a.n_head < 1024;
+    const unsigned wgs = (unsigned)(split ? n_groups : (n_groups + 3) / 4), heads = (unsigned)a.n_head;
+    hipLaunchKernelGGL((split ? t3_attn_tile<4> : t3_attn_tile<1>),
+                       a.rows ? dim3(heads, wgs) : dim3(wgs, heads), dim3(4 * kHeadDim), 0, st, a,
+                       n_rows, n_groups);
     return hipGetLastError();
 }
 
@@ -808,13 +823,6 @@ size_t t3_attn_lds(int32_t) { return 0; }  // one pass: no per-position LDS
 // workgroups and merged by a second kernel).
 bool t3_attn_wide(int32_t n_rows, int32_t n_head) { return (int64_t)n_rows * n_head < 256; }
 
-// Workspace of a step: x, u, a [n_rows][n_embd], y [kMaxKSplit][n_rows][n_embd],
-// qkv [n_rows][3 n_embd], f [n_rows][4 n_embd], act [n_rows], then two
-// buffers of split activations for the matrix products (each for the widest
-// input, 4 n_embd): the norms and the attention write the first, the mlp's
-// c_fc the second (c_fc reads the first as it writes), then, where the rows are
-// many (head_uses_tiles), the largest matrix unpacked for its product.
-
 // Streams on the matrix cores, every product's input written split by its
 // producer; fewer run the mat-vecs on plain rows.  us per step of the Turbo
 // shape at position 256, mat-vecs / matrix cores: Q4_0 4 streams 1146 / 1012, 6
@@ -830,12 +838,23 @@ static size_t t3_split_bytes(int32_t n_rows, int32_t n_embd) {
     return (split_bytes((n_rows + 15) / 16 * 16, 4 * n_embd) + 255) / 256 * 256;
 }
 
+// Bytes of the prompt pass's row groups (group_bound: at most n_rows of them).
+static size_t t3_group_bytes(int32_t n_rows) { return ((size_t)n_rows * 64 + 255) / 256 * 256; }
+
+// Workspace of a step: x, u, a [n_rows][n_embd], y [kMaxKSplit][n_rows][n_embd],
+// qkv [n_rows][3 n_embd], f [n_rows][4 n_embd], act [n_rows], then two
+// buffers of split activations for the matrix products (each for the widest
+// input, 4 n_embd): the norms and the attention write the first, the mlp's
+// c_fc the second (c_fc reads the first as it writes), then the prompt pass's
+// row groups and, where the rows are many (head_uses_tiles), the largest matrix
+// unpacked for its product.
 size_t t3_workspace_bytes(int32_t n_rows, int32_t n_embd) {
     const size_t row = (size_t)n_rows * n_embd * 4;
     const size_t body = (3 + kMaxKSplit) * row + 3 * row + 4 * row +
                         ((size_t)n_rows * 4 + 255) / 256 * 256;
-    return body + 2 * t3_split_bytes(n_rows, n_embd) + max(tile_scratch_bytes(n_rows, 4 * n_embd, n_embd),
-                               tile_scratch_bytes(n_rows, n_embd, 4 * n_embd));
+    return body + 2 * t3_split_bytes(n_rows, n_embd) + t3_group_bytes(n_rows) +
+           max(tile_scratch_bytes(n_rows, 4 * n_embd, n_embd),
+               tile_scratch_bytes(n_rows, n_embd, 4 * n_embd));
 }
 
 hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* tokens,
@@ -857,7 +876,9 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     const bool wide = !prefill && t3_attn_wide(n_rows, m.n_head);
     void* split = reinterpret_cast<char*>(act) + ((size_t)n_rows * 4 + 255) / 256 * 256;
     void* split2 = static_cast<char*>(split) + t3_split_bytes(n_rows, n);
-    void* unpacked = static_cast<char*>(split2) + t3_split_bytes(n_rows, n);
+    int32_t* const groups =
+        reinterpret_cast<int32_t*>(static_cast<char*>(split2) + t3_split_bytes(n_rows, n));
+    void* unpacked = reinterpret_cast<char*>(groups) + t3_group_bytes(n_rows);
 
     NormArgs na{};
     na.n_embd = n;
@@ -904,6 +925,16 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
     aa.inv = sinv;
     aa.scale = 0.125f;  // 1 / sqrt(64)
     const size_t lds = t3_attn_lds(c.n_ctx);
+    // the prompt pass's rows in groups of one slot each (one row or one slot
+    // is grouped as it is)
+    int n_groups = (n_rows + 15) / 16;
+    if (prefill && n_rows > 1 && n_slots > 1) {
+        n_groups = group_bound(n_rows, n_slots);
+        aa.rows = groups;
+        hipLaunchKernelGGL(t3_group_rows, dim3(1), dim3(kGroupThreads), 0, st, act, slots, n_rows,
+                           n_groups, groups);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
 
     const int kz_a = mc ? min(head_k_split(n_rows, n, n), kMaxKSplit) : 1;
     const int kz_f = mc || !head_uses_gemv(n_rows, false, 4 * n)
@@ -955,7 +986,7 @@ hipError_t launch_t3_step(const cbx_t3_model& m, int32_t n_rows, const int32_t* 
                                    dim3(kHeadDim), 0, st, aa);
                 if ((e = hipGetLastError()) != hipSuccess) return e;
             }
-            if ((e = launch_attn_tile(aa, n_rows, st)) != hipSuccess) return e;
+            if ((e = launch_attn_tile(aa, n_rows, n_groups, st)) != hipSuccess) return e;
         } else if (wide) {
             hipLaunchKernelGGL((t3_attn<6, 16>), dim3((unsigned)n_rows, (unsigned)m.n_head),
                                dim3(16 * kHeadDim), lds, st, aa);

@@ -20,6 +20,7 @@ def lib():
         L = ctypes.CDLL(LIB)
         vp, i64 = ctypes.c_void_p, ctypes.c_int64
         L.cbx_debug_t3_gelu.argtypes = [vp, vp, i64, vp]
+        L.cbx_debug_t3_groups.argtypes = [vp, vp, ctypes.c_int32, ctypes.c_int32, vp, vp]
         _lib = L
     return _lib
 
@@ -36,3 +37,15 @@ def _ok(rc, name):
 
 def gelu(x, out):
     _ok(lib().cbx_debug_t3_gelu(x.data_ptr(), out.data_ptr(), x.numel(), _stream()), "gelu")
+
+
+def groups(act, slots, n_slots):
+    """t3_group_rows on device int32 act and slots: [groups, 16] row numbers, -1 for none."""
+    import torch
+    n = slots.numel()
+    G = lib().cbx_debug_t3_groups(None, None, n, n_slots, None, None)
+    rows = torch.full((G, 16), -7, dtype=torch.int32, device=slots.device)
+    if lib().cbx_debug_t3_groups(act.data_ptr(), slots.data_ptr(), n, n_slots, rows.data_ptr(),
+                                 _stream()) != G:
+        raise RuntimeError("groups failed")
+    return rows

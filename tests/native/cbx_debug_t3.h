@@ -15,6 +15,11 @@ extern "C" {
 /* The T3 MLP's gelu (t3_gelu_f, cbx_split.h), elementwise. */
 int cbx_debug_t3_gelu(const float* in, float* out, int64_t n, void* stream);
 
+/* The prompt pass's row groups (t3_group_rows, cbx_group.h): returns their
+ * bound G; with rows set, 16 G row numbers or -1 are written there. */
+int cbx_debug_t3_groups(const int32_t* act, const int32_t* slots, int32_t n_rows, int32_t n_slots,
+                        int32_t* rows, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -277,3 +277,66 @@ def test_split_norm_widths(small, n_head):
         torch.cuda.synchronize()
         want = T3.step(rm, toks, at, kr, vr, active=state == 0)
         assert np.all(np.abs(hid.cpu().numpy() - want) <= TOL_ABS + TOL_REL * np.abs(want))
+
+
+GROUPED = [(1, 1), (2, 2), (3, 3), (17, 2), (64, 64), (251, 64), (1000, 7), (4096, 4096),
+           (5000, 1), (5001, 4097), (14975, 64), (20000, 9000)]
+
+
+@pytest.mark.parametrize("order", ["random", "runs", "interleaved"])
+@pytest.mark.parametrize("n,n_slots", GROUPED, ids=[f"{n}-{b}" for n, b in GROUPED])
+def test_row_groups(small, n, n_slots, order):
+    """t3_group_rows (csrc/cbx_group.h): every row in one group, a group's rows
+    of one slot (modulo 4096) or all skipped, in the caller's order, at most 15
+    places empty per slot; nothing written past the bound."""
+    import debug_t3_lib as D
+    torch = small[0]
+    rng = np.random.default_rng(n + n_slots)
+    slots = {"random": rng.integers(0, n_slots, n), "runs": np.arange(n) * n_slots // n,
+             "interleaved": np.arange(n) % n_slots}[order].astype(np.int32)
+    act = (rng.random(n) < 0.9).astype(np.int32)
+    slots[act == 0] = rng.choice([-5, 2 ** 31 - 1], int((act == 0).sum()))
+    print(f"[gpu-case] groups {n} rows {n_slots} slots {order}", flush=True)
+    got = D.groups(torch.from_numpy(act).cuda(), torch.from_numpy(slots).cuda(), n_slots)
+    got = got.cpu().numpy()
+    assert got.shape[0] <= min(n, n // 16 + min(n_slots, 4096) + 1)
+    assert np.array_equal(np.sort(got[got >= 0]), np.arange(n)) and got.min() >= -1
+    key = np.where(act != 0, slots & 4095, 4096)
+    last = {}
+    for g in got:
+        rows = g[g >= 0]
+        if rows.size == 0:
+            continue
+        assert np.array_equal(g[: rows.size], rows)  # the empty places last
+        k = set(key[rows].tolist())
+        assert len(k) == 1
+        k = k.pop()
+        assert k not in last or (last[k][1] == 16 and last[k][0] < rows[0])
+        assert np.all(np.diff(rows) > 0)
+        last[k] = (rows[-1], rows.size)
+
+
+@pytest.mark.parametrize("B,L,n_slots", [(2, 30, 2), (3, 40, 3), (20, 33, 20), (300, 20, 300),
+                                         (24, 9, 8200)])
+def test_one_row_per_stream(small, B, L, n_slots):
+    """A call of one row per stream after their prompts: the rows of a mixed
+    group, each over its own stream's positions, and 2 and 3 rows (mat-vecs, keys
+    and values stored by t3_kv_append) in two and three slots.  8200 slots: some
+    rows of one group in slots equal modulo 4096."""
+    torch, s, dm, rm = small
+    rng = np.random.default_rng(B)
+    at = np.arange(B) if n_slots == B else np.concatenate(
+        [[b, b + 4096, b + 8192] for b in range(B // 3)])
+    x = {(b, p): (rng.standard_normal(N) * 0.7).astype(np.float32)
+         for b in range(B) for p in range(L)}
+    print(f"[gpu-case] one row per stream B={B} L={L} slots={n_slots}", flush=True)
+    first = [(b, p) for p in range(L - 1) for b in range(B)]
+    last = [(b, L - 1) for b in range(B)]
+    place = lambda rows: [(int(at[b]), p) for b, p in rows]
+    _, k, v = run(torch, s, dm, place(first), np.stack([x[r] for r in first]), n_slots, L)
+    got, _, _ = run(torch, s, dm, place(last), np.stack([x[r] for r in last]), n_slots, L, (k, v))
+    for b in range(0, B, max(1, B // 24)):
+        kr, vr = T3.new_cache(1, L_, H, L)
+        want = T3.prefill(rm, np.stack([x[(b, p)] for p in range(L)]), kr, vr, 0, 0)[-1]
+        err = np.abs(got[b] - want)
+        assert np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), f"stream {b}: {err.max():.3g}"
