@@ -301,10 +301,14 @@ int cbx_sample_row_ex(cbx_sampler* s, const float* logits, const float* logits_u
     a.info = &ds->info;
     a.probs = probs_out ? s->d_probs : nullptr;
     a.ld_probs = n_vocab;
-    CBX_HIP(launch_with_redo(pick_cap(s, n_vocab, 0), a, s->d_redo_row, s->latency_rows, st));
-    if (probs_out)
-        CBX_HIP(hipMemcpyAsync(probs_out, s->d_probs, sizeof(float) * n_vocab, hipMemcpyDeviceToHost, st));
-    CBX_HIP(hipStreamSynchronize(st));
+    hipError_t e = launch_with_redo(pick_cap(s, n_vocab, 0), a, s->d_redo_row, s->latency_rows, st);
+    if (e == hipSuccess && probs_out)
+        e = hipMemcpyAsync(probs_out, s->d_probs, sizeof(float) * n_vocab, hipMemcpyDeviceToHost, st);
+    // where that failed too: a kernel already launched reads the pinned
+    // buffers, which the next call writes
+    const hipError_t done = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = done;
+    if (e != hipSuccess) return fail(CBX_ERR_HIP, "cbx_sample_row: %s", hipGetErrorString(e));
     *token_out = hs->token;
     if (info_out) *info_out = hs->info;
     if (hs->info & CBX_INFO_OVERFLOW)
