@@ -489,9 +489,9 @@ int check_head(const char* fn, const cbx_head* h, int32_t n_rows, int32_t n_voca
 }
 
 // The handle's split buffer holds one call's activations at a time: head calls
-// of 16 projected rows and more on one handle are ordered on one stream (a
-// larger call than any before waits for the device while the buffer is
-// replaced); smaller ones do not use it.
+// of 16 projected rows (or more than 62 KiB of them) on one handle are ordered on
+// one stream (a larger call than any before waits for the device while the
+// buffer is replaced); smaller ones do not use it.
 int run_head(cbx_sampler* s, const cbx_head* h, int32_t n_rows, int32_t n_vocab,
              int64_t ld_logits, hipStream_t st) {
     const size_t need = cbx::head_scratch_bytes(n_rows, h->hidden_uncond != nullptr, h->n_embd);

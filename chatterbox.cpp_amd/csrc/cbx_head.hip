@@ -145,7 +145,7 @@ constexpr int RING = 2;
 // (rows of n_vocab values: this workgroup's 32 outputs are block blockIdx.x
 // of each of its rows) instead of fp32 rows.
 // KV: a q|k|v product, its k and v stored in the caches (kv_place).
-// SELF (at most 15 rows: one tile per row set): the rows themselves (`rows`)
+// SELF (head_holds_nothing; one tile per row set): the rows themselves (`rows`)
 // instead of their split; a block's values are split as the block is taken, by
 // the operations of head_split and with the same results.  The split (about 70
 // VALU instructions per block) is repeated by every workgroup, but no launch
@@ -882,17 +882,20 @@ hipError_t mfma_dispatch(const void* W, int32_t wtype, const float* bias, const 
 // cores, the others within 0.2).  Up to 6 rows the activations stay fp32
 // operands (a guided batch of 3 and fewer), so their results are the mat-vec's.
 bool head_uses_gemv(int32_t n_rows, bool cfg, int32_t n_embd) {
-    const int R = cfg ? 2 * n_rows : n_rows;
-    return R < 7 && (size_t)R * gemv_row_words(n_embd) * 4 <= 65536;
+    return (cfg ? 2 * n_rows : n_rows) < 7 && head_holds_nothing(n_rows, cfg, n_embd);
 }
 
-// Calls of fewer projected rows hold nothing in memory between launches, so
-// they may run on several streams of one handle at once.
-constexpr int kSelfRows = 16;
+// The split inside the product is repeated by every workgroup, for the whole of
+// n_embd: longer rows take the launch before it (us per call at V = 6563, Q4_0,
+// split launch / inside: 7 rows of n_embd 4096 15.3 / 17.7, of 16384 48.9 / 68.5).
+bool head_holds_nothing(int32_t n_rows, bool cfg, int32_t n_embd) {
+    const int R = cfg ? 2 * n_rows : n_rows;
+    return R < 16 && (size_t)R * gemv_row_words(n_embd) * 4 <= 65536;
+}
 
 size_t head_scratch_bytes(int32_t n_rows, bool cfg, int32_t n_embd) {
     const int n_tiles = ((n_rows + 15) / 16) * (cfg ? 2 : 1);
-    return n_rows * (cfg ? 2 : 1) < kSelfRows ? 0 : split_bytes(16 * n_tiles, n_embd);
+    return head_holds_nothing(n_rows, cfg, n_embd) ? 0 : split_bytes(16 * n_tiles, n_embd);
 }
 
 hipError_t launch_head(const void* W, int32_t wtype, const float* bias, const float* hidden0,
@@ -917,7 +920,7 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
                          void* scratch, hipStream_t stream, int kz, bool gelu_out) {
     // fewer than 7 projected rows: the mat-vec (activations staged in LDS,
     // at most 64 KiB of them), else the 16-row matrix-core tiles, from 16
-    // projected rows after a launch that splits them
+    // projected rows (or longer ones) after a launch that splits them
     const bool cfg = hidden1 != nullptr;
     if (kz < 1 || (kz > 1 && (cfg || gelu_out || head_uses_gemv(n_rows, cfg, n_embd))))
         return hipErrorInvalidValue;  // a K split: one row set on the matrix cores, no gelu
@@ -944,7 +947,7 @@ hipError_t launch_head_k(const void* W, int32_t wtype, const float* bias, const 
         }
     }
     const int n_tiles = ((n_rows + 15) / 16) * (cfg ? 2 : 1), R = 16 * n_tiles;
-    if (n_rows * (cfg ? 2 : 1) < kSelfRows)
+    if (head_holds_nothing(n_rows, cfg, n_embd))
         return mfma_dispatch(W, wtype, bias, nullptr, nullptr, n_tiles, out0, out1, ld_out, n_rows,
                              n_vocab, n_embd, stream, kz, gelu_out ? 1 : 0, nullptr, nullptr,
                              KvOut{}, HeadRows{hidden0, hidden1, ld_hidden});

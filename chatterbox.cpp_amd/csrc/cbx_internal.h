@@ -118,8 +118,8 @@ hipError_t launch_decode_v1024x32(const KernelArgs& a, hipStream_t stream);
 // for r < n_rows, v < n_vocab, and the same from hidden1 into out1 in the same
 // launches when hidden1 is given.  `scratch` is device memory of at least
 // head_scratch_bytes(n_rows, hidden1 != NULL, n_embd) bytes (the activations
-// split for the matrix cores; 0 bytes, and NULL allowed, below 16 projected
-// rows).
+// split for the matrix cores; 0 bytes, and NULL allowed, where
+// head_holds_nothing).
 size_t head_scratch_bytes(int32_t n_rows, bool cfg, int32_t n_embd);
 // Bytes per block of 32 weights of a CBX_WTYPE_* (0 for an unknown type).
 inline int64_t wtype_block_bytes(int32_t wtype) {
@@ -131,6 +131,10 @@ inline int64_t wtype_block_bytes(int32_t wtype) {
         default: return 0;
     }
 }
+// Whether launch_head keeps nothing in memory between launches (fewer than 16
+// projected rows, 62 KiB of them at most): such calls may run on several
+// streams of one handle at once.
+bool head_holds_nothing(int32_t n_rows, bool cfg, int32_t n_embd);
 // Whether launch_head takes the mat-vec (fewer than 7 projected rows whose
 // activations fit its LDS) rather than the matrix cores.
 bool head_uses_gemv(int32_t n_rows, bool cfg, int32_t n_embd);

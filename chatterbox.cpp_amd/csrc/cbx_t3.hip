@@ -832,9 +832,10 @@ static bool t3_matrix(int32_t n_rows, int32_t n_embd) {
     return n_rows >= 4 || !head_uses_gemv(n_rows, false, n_embd);
 }
 
-// Bytes of one split buffer of the widest input.
+// Bytes of one split buffer of the widest input (also where the mat-vecs'
+// LDS cannot hold rows of 4 n_embd).
 static size_t t3_split_bytes(int32_t n_rows, int32_t n_embd) {
-    if (!t3_matrix(n_rows, n_embd)) return 0;
+    if (!t3_matrix(n_rows, n_embd) && head_uses_gemv(n_rows, false, 4 * n_embd)) return 0;
     return (split_bytes((n_rows + 15) / 16 * 16, 4 * n_embd) + 255) / 256 * 256;
 }
 

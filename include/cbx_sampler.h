@@ -211,10 +211,11 @@ typedef struct cbx_head {
  * on (cond and uncond rows together; fewer where n_embd is too long for the
  * mat-vec's LDS), the fp16 matrix cores take each activation, scaled by a power
  * of two per 32 of its row, as two fp16 parts (to 2^-23 relative plus 2^-39 of
- * the largest magnitude among the 32).  From 16 projected rows on, these are
- * held in a device buffer of the handle that a call larger than any before it
- * replaces (waiting for the device): such calls on one handle are ordered on
- * one stream.  Smaller calls hold nothing in the handle.
+ * the largest magnitude among the 32).  From 16 projected rows on, and where
+ * the projected rows are more than 62 KiB, these are held in a device buffer of
+ * the handle that a call larger than any before it replaces (waiting for the
+ * device): such calls on one handle are ordered on one stream.  Smaller calls
+ * hold nothing in the handle.
  * Replaces the speech_head mul_mat of the T3 step (main.cpp:577).  Async. */
 int cbx_head_logits(cbx_sampler* s, const cbx_head* h, int32_t n_rows, int32_t n_vocab,
                     int64_t ld_logits, void* stream);
