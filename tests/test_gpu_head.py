@@ -80,15 +80,16 @@ CASES = [
     (O.WTYPE_Q4_0, 8194, 1024, 2, 8194),     # one CFG pair, the Llama vocab
     (O.WTYPE_Q8_0, 300, 64, 17, 301),        # ragged tiles on both axes
     (O.WTYPE_F16, 33, 32, 1, 40),
-    # fewer than 16 rows: the mat-vec kernel
+    # fewer than 7 rows: the mat-vec kernel (15: the largest call that splits
+    # its rows inside the product)
     (O.WTYPE_Q4_0, 6563, 1024, 1, 6563),     # one stream of the Turbo vocab
     (O.WTYPE_Q8_0, 6563, 1024, 2, 6570),
     (O.WTYPE_F16, 6563, 1024, 2, 6563),
-    (O.WTYPE_Q4_0, 6563, 1024, 15, 6563),    # the largest mat-vec batch
+    (O.WTYPE_Q4_0, 6563, 1024, 15, 6563),
     (O.WTYPE_Q8_0, 1000, 4096, 3, 1000),
     (O.WTYPE_Q4_0, 300, 64, 5, 301),
     (O.WTYPE_F16, 500, 8192, 1, 500),
-    (O.WTYPE_Q4_0, 700, 512, 16, 700),       # 16 rows: the matrix-core tiles again
+    (O.WTYPE_Q4_0, 700, 512, 16, 700),       # 16 rows: split by a launch before the product
     (O.WTYPE_Q5_0, 6563, 1024, 128, 6563),   # Q5_0 (--quant q5_0): the matrix cores
     (O.WTYPE_Q5_0, 300, 64, 17, 301),        #   ragged tiles on both axes
     (O.WTYPE_Q5_0, 6563, 1024, 2, 6563),     #   the mat-vec, one CFG pair
@@ -184,8 +185,8 @@ def test_fused_head_sample_cfg(cbx, torch_cuda, wtype, B, S):
     """B CFG streams, S steps: projection of cond and uncond hidden rows
     (weights from N(0, 0.02), hidden rows N(0, 1)), then the sampler (k 1000,
     p 0.95, T 0.8, pen 1.2, w 0.5) in one call.  B=64 x 2 projects 256 rows
-    on the matrix cores; one CFG pair (2 rows) and 7 pairs (14 rows) take the
-    mat-vec kernel."""
+    on the matrix cores after a split launch, 7 pairs (14 rows) split theirs in
+    the product; one CFG pair (2 rows) takes the mat-vec kernel."""
     torch = torch_cuda
     mod, s = cbx
     V, K = 6563, 1024

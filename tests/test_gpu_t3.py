@@ -106,15 +106,15 @@ def close(got, want):
     return np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), float(err.max())
 
 
-@pytest.mark.parametrize("B", [20, 5, 2, 1])
+@pytest.mark.parametrize("B", [20, 5, 3, 2, 1])
 @pytest.mark.parametrize("wtype", [O.WTYPE_Q4_0, O.WTYPE_Q5_0, O.WTYPE_Q8_0, O.WTYPE_F16])
 def test_t3_step_matches_oracle(cbx, torch_cuda, wtype, B):
     """B streams, 4 steps with per-stream ids; in step 2 every third stream
     sits out (state not running), so positions differ afterwards.  Each step's
     ln_f rows, every stream's position and the skipped rows' zeros match the
-    oracle.  B = 20 runs the products on the matrix cores, B = 5 on the
-    mat-vec; B = 2 and 1 fold the residual adds and norms between a layer's
-    products into the mat-vec that consumes them."""
+    oracle.  B = 20 and 5 run the products on the matrix cores (two row tiles
+    and one), B = 3 on the mat-vec; B = 2 and 1 fold the residual adds and norms
+    between a layer's products into the mat-vec that consumes them."""
     torch = torch_cuda
     mod, s = cbx
     dm, rm = model(torch, mod, wtype)
@@ -333,14 +333,14 @@ def test_t3_from_gguf(cbx, torch_cuda, tmp_path, B, wtype):
         assert ok, f"step {t}: max err {err:.3g}"
 
 
-@pytest.mark.parametrize("lens", [(5, 9, 7), (2, 3)])
+@pytest.mark.parametrize("lens", [(5, 9, 7), (2, 3), (1, 2), (3,), (1, 1)])
 def test_t3_prefill_then_decode(cbx, torch_cuda, lens):
     """Prompts of several streams in one cbx_t3_prefill call (rows in shuffled
     order, embedded input rows), then two cbx_t3_step decode steps: every
     prompt row's ln_f output matches the oracle stepping each stream through
     its positions one at a time (the causal prompt pass), and the decode
-    steps continue from the caches the prefill wrote.  21 rows take the
-    matrix cores, 5 the mat-vec."""
+    steps continue from the caches the prefill wrote.  21 and 5 rows take the
+    matrix cores; up to 3 the mat-vec, a launch storing their keys and values."""
     torch = torch_cuda
     mod, s = cbx
     dm, rm = model(torch, mod, O.WTYPE_Q4_0)
@@ -413,6 +413,7 @@ def host_caches(kd, vd, lengths):
 LONG_POSITIONS = {
     16: [0, 1, 95, 96, 97, 98, 191, 200, 385, 500, 777, 1000, 1500, 2047, 3001, N_CTX_LONG - 1],
     5: [384, 385, 1000, 2500, 4000],
+    3: [384, 1001, 4000],
     1: [N_CTX_LONG - 2],
 }
 
@@ -424,8 +425,8 @@ def test_t3_step_long_context(cbx, torch_cuda, B):
     planted, several positions per call; then a second step, where a stream
     at n_ctx - 1 has run out of cache and sits out (zero row, position
     unchanged).  16 streams run the 4-wave attention and the matrix cores,
-    5 the 16-wave attention and the mat-vec, 1 the 16-wave attention and the
-    mat-vec with folded norms."""
+    5 the 16-wave attention and the matrix cores, 3 the 16-wave attention and
+    the mat-vec, 1 the 16-wave attention and the mat-vec with folded norms."""
     torch = torch_cuda
     mod, s = cbx
     dm, rm = model(torch, mod, O.WTYPE_Q4_0, n_pos=N_CTX_LONG)
@@ -459,8 +460,8 @@ def test_t3_step_long_context(cbx, torch_cuda, B):
 
 
 def test_t3_prefill_long_then_decode(cbx, torch_cuda):
-    """The prompt pass at lengths where the 2-wave prompt attention runs
-    several batches per wave: stream 0's 320-position prompt from position
+    """The prompt pass at lengths where each wave of the prompt attention
+    takes several pairs of key tiles: stream 0's 320-position prompt from position
     0, and stream 1's 130 rows continuing a planted 150-position cache (a
     prompt fed in two calls), 450 rows shuffled in one cbx_t3_prefill call
     (matrix cores), against the oracle's one-pass prompt; then two decode
