@@ -105,6 +105,11 @@ __device__ __forceinline__ i4 buffer(const void* p, int64_t bytes) {
 // the builtins the compiler waits for all of them before any LDS read, and
 // the point is to keep later blocks' loads in flight.  No register is
 // written; the waits are wait_stage's.
+// (-Winline-asm: that m0 is a reserved register, which holds a load's LDS base
+// and is set right before each; the compiler sets it anew for its own uses, told
+// by the clobber.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, const i4& rsrc, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
@@ -113,6 +118,7 @@ __device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, const i4& rsrc
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
                  ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // This wave's loads but the last N done, its LDS reads too; then the others'.
 template <int N>
 __device__ __forceinline__ void wait_stage() {

@@ -77,47 +77,6 @@ __device__ __forceinline__ f4 mfma_f16(const u4v& a, const u4v& b, const f4& c) 
                                                   __builtin_bit_cast(h8, b), c, 0, 0, 0);
 }
 
-// A 16-row x 32-output product tile as block `blk` of the next product's
-// split rows (cbx_split.h; nb_out blocks a row): lane (g, m) holds rows
-// 4g + i of tile T at outputs m (xa) and 16 + m (xb).  A row's largest
-// magnitude comes from its 16 lanes, then lane (g, m) holds the values of
-// group m / 8 (output m) and group 2 + m / 8 (output 16 + m) at place m % 8;
-// pairs of lanes join their halves into dwords.  Nothing stored unless `in`.
-__device__ __forceinline__ void store_split_tile(uint32_t* out_parts, float* out_inv, int T, bool in,
-                                                 int nb_out, int blk, int g, int m,
-                                                 const float (&xa)[4], const float (&xb)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float mx = fmaxf(fabsf(xa[i]), fabsf(xb[i]));
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        float scl, sinv;
-        split_scale(mx, scl, sinv);
-        const float ya = __fmul_rn(xa[i], scl), yb = __fmul_rn(xb[i], scl);
-        const _Float16 ha = (_Float16)ya, hb = (_Float16)yb;
-        const _Float16 la = (_Float16)__fsub_rn(ya, (float)ha);
-        const _Float16 lb = (_Float16)__fsub_rn(yb, (float)hb);
-        // the odd lane's halves join the even lane's dword
-        const uint32_t hab = (uint32_t)__builtin_bit_cast(uint16_t, ha) |
-                             (uint32_t)__builtin_bit_cast(uint16_t, hb) << 16;
-        const uint32_t lab = (uint32_t)__builtin_bit_cast(uint16_t, la) |
-                             (uint32_t)__builtin_bit_cast(uint16_t, lb) << 16;
-        const uint32_t hab_o = (uint32_t)__shfl_xor((int)hab, 1);
-        const uint32_t lab_o = (uint32_t)__shfl_xor((int)lab, 1);
-        const int mrow = 4 * g + i;  // the row's place in its tile
-        if (in && (m & 1) == 0) {
-            // dword (m % 8) / 2 of lane 16 gq + mrow's hi (lo) 16 bytes
-            uint32_t* const base = out_parts + ((int64_t)T * nb_out + blk) * 512 + (m & 7) / 2;
-            const int ga = m >> 3, gb = 2 + (m >> 3);
-            base[4 * (16 * ga + mrow)] = (hab & 0xffffu) | (hab_o << 16);
-            base[4 * (16 * ga + mrow) + 256] = (lab & 0xffffu) | (lab_o << 16);
-            base[4 * (16 * gb + mrow)] = (hab >> 16) | (hab_o & 0xffff0000u);
-            base[4 * (16 * gb + mrow) + 256] = (lab >> 16) | (lab_o & 0xffff0000u);
-        }
-        if (in && m == 0) out_inv[split_inv_index(T, mrow, nb_out, blk)] = sinv;
-    }
-}
-
 // Where k or v of row r, column v >= n of a q|k|v product of n columns each
 // goes (NULL: nowhere); every 32 columns from a multiple of 32 lie in one head.
 __device__ __forceinline__ float* kv_place(const KvOut& kv, int r, int v) {
