@@ -553,9 +553,10 @@ __global__ __launch_bounds__(kAttnWaves * kHeadDim) void t3_attn(AttnArgs a) {
 // pair of tiles, merged through LDS by the same rescaling in wave order
 // (small calls); KS = 1: each wave its own rows.
 // Measured per layer at 64 prompts of 129 to 383 rows (14975 in all), 16
-// heads: 1051 -> 200 us (matrix cores busy 42% of it; they alone would take
-// about 80); one prompt of 251 rows 24.5 -> 11 us.  32 rows per wave (half the
-// loads of K and V) measured 235: registers for two waves per SIMD, not three.
+// heads: 1051 -> 175 us (matrix cores busy 35% of its cycles, VALU 34%; ready
+// waves that another is issued before, 47% of the waves' time); one prompt of 251
+// rows 24.5 -> 9.4 us.  32 rows per wave (half the loads of K and V) measured 235,
+// where this took 200: registers for two waves per SIMD, not three.
 template <int KS>
 __global__ __launch_bounds__(4 * kHeadDim) void t3_attn_tile(AttnArgs a, int n_rows,
                                                             int n_groups) {
@@ -826,8 +827,10 @@ bool t3_attn_wide(int32_t n_rows, int32_t n_head) { return (int64_t)n_rows * n_h
 // Streams on the matrix cores, every product's input written split by its
 // producer; fewer run the mat-vecs on plain rows.  us per step of the Turbo
 // shape at position 256, mat-vecs / matrix cores: Q4_0 4 streams 1146 / 1012, 6
-// 1381 / 1052, 8 1497 / 1050, 15 2128 / 1115; Q8_0 6 1406 / 1107.  (3 streams,
-// 1153 / 982, stay: their rows are bit for bit those of one or two.)
+// 1381 / 1052, 8 1497 / 1050, 15 2128 / 1115; Q8_0 6 1406 / 1107.  3 streams,
+// 1153 / 982, stay on the mat-vecs all the same: their activations stay fp32
+// operands, and a stream's rows are bit for bit what they are beside one other
+// or alone (the folded norms are checked against the separate ones there).
 static bool t3_matrix(int32_t n_rows, int32_t n_embd) {
     return n_rows >= 4 || !head_uses_gemv(n_rows, false, n_embd);
 }

@@ -9,12 +9,17 @@
 // neither shift nor convert them again (about 80 VALU instructions per block
 // and wave); head_tile multiplies.
 // Measured, 14975 rows of the Turbo shape (Q4_0, us, head_mfma -> here): c_fc with
-// gelu and split outputs 697 -> 305, the layer's other three 1146 -> 554 (c_attn
-// 203, attn c_proj 76, mlp c_proj 275), unpacking 21; the prompt pass of 64 x
-// 129-383 rows 53.6 -> 31.6 ms.  The products run twice (hi, lo): 18.1 TFLOP, 875
-// TFLOP/s; a library product of 8192^3 in fp16 reaches 1174 on this card.
-// What bounds it: the VALU's scaled adds (8 per tile beside 2 matrix products)
-// and the matrix cores together fill about 85% of a SIMD's cycles.
+// gelu and split outputs 697 -> 317, the layer's other three 1146 -> 590 (c_attn
+// 234, the two c_proj 356), unpacking 25; the prompt pass of 64 x 129-383 rows
+// 53.6 -> 31.6 ms.  The products run twice (hi, lo): 18.1 TFLOP, 830 TFLOP/s; a
+// library product of 8192^3 in fp16 reaches 1174 on this card.
+// What bounds it (counters, of a SIMD's cycles): the matrix cores are busy 36-40%,
+// VALU instructions (theirs included) issue in 60% (c_proj) to 81% (c_fc); there
+// are no bank conflicts outside the split outputs, and a wave spends a third of
+// its time ready but not issued, a third waiting.  F16, without the weights'
+// scales, issues 46-70%, its matrix cores are busy 41-47%, in 11-14% fewer cycles:
+// the shared issue of scaled adds and matrix products bounds it, with the waits
+// at the barrier of each block next.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -78,8 +78,11 @@ typedef struct cbx_t3_cache {
  * skipped (nothing written to its cache, its hidden row zero, its position
  * unchanged) when state is given and state[r] != CBX_DECODE_RUNNING, when
  * its position is outside [0, cache.n_ctx) or its token outside
- * [0, n_speech_vocab).  Asynchronous on `stream`; the handle holds the
- * step's workspace (grown on demand: calls on one handle are ordered on one
+ * [0, n_speech_vocab).  Sums are fp32; from 4 streams on, the products run on
+ * the fp16 matrix cores, which take each of their input rows' values, scaled by
+ * a power of two per 32, as two fp16 parts (to 2^-23 relative plus 2^-39 of the
+ * largest magnitude among the 32), fewer streams' inputs as they are.
+ * Asynchronous on `stream`; the handle holds the step's workspace (grown on demand: calls on one handle are ordered on one
  * stream).  Replaces eval_step (main.cpp:691-710) up to ln_f for every
  * stream at once. */
 int cbx_t3_step(cbx_sampler* s, const cbx_t3_model* m, int32_t n_rows,
@@ -99,7 +102,9 @@ int cbx_t3_step(cbx_sampler* s, const cbx_t3_model* m, int32_t n_rows,
  * row's position already in the cache or in the call.  ln_f's rows go to
  * hidden[r]; positions are only read.  Rows whose slot is outside
  * [0, n_slots), position outside [0, cache.n_ctx) or token outside
- * [0, n_speech_vocab) are skipped.  The cache holds n_slots streams.
+ * [0, n_speech_vocab) are skipped.  The cache holds n_slots streams.  Rows may
+ * come in any order (they are grouped by slot on the device); from 4 rows on the
+ * products take their inputs in two fp16 parts as cbx_t3_step's do.
  * Asynchronous on `stream`.  Replaces eval_prompt (main.cpp:643-689) up to
  * ln_f, for any number of streams at once. */
 int cbx_t3_prefill(cbx_sampler* s, const cbx_t3_model* m, int32_t n_rows,

@@ -340,3 +340,29 @@ def test_one_row_per_stream(small, B, L, n_slots):
         want = T3.prefill(rm, np.stack([x[(b, p)] for p in range(L)]), kr, vr, 0, 0)[-1]
         err = np.abs(got[b] - want)
         assert np.all(err <= TOL_ABS + TOL_REL * np.abs(want)), f"stream {b}: {err.max():.3g}"
+
+
+def test_captured_prompt(small):
+    """A prompt call of mixed slots captured in a graph and replayed, other
+    prompts run between the replays, gives the eager call's rows."""
+    torch, s, dm, _ = small
+    rng = np.random.default_rng(21)
+    rows = arranged((30, 7, 41, 1), "positions", rng)
+    at = np.array(rows, np.int32)
+    t = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    slots, pos = t(at[:, 0].copy()), t(at[:, 1].copy())
+    x = t((rng.standard_normal((len(rows), N)) * 0.7).astype(np.float32))
+    want, k, v = run(torch, s, dm, rows, x.cpu().numpy(), 4, 64)
+    hid = torch.zeros_like(x)
+    print("[gpu-case] captured prompt", flush=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        s.t3_prefill(dm, slots, pos, k, v, hid, inputs=x)
+    for _ in range(3):
+        run(torch, s, dm, rows[:50], np.ones((50, N), np.float32), 4, 64)
+        k.fill_(float("nan"))
+        v.fill_(float("nan"))
+        hid.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(hid.cpu().numpy(), want)
